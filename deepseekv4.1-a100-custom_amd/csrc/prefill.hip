@@ -43,6 +43,7 @@ struct PrefillArgs {
     int cbw, n_it;                            // column blocks per workgroup, workgroups per group (ceil(n_cb / cbw))
     const int* run_if;                        // MODE 2, optional: the launch does nothing when *run_if == 0
     const int* grp_order;                     // optional: the order the items take the groups in (dsv41_group_order)
+    int g_max;                                // light tile: pairs of a group that are computed
 };
 
 // The group an item's group index stands for: the index itself, or its place in grp_order (largest groups first, so no
@@ -113,6 +114,40 @@ template <int N>
 struct IntC {
     static constexpr int value = N;
 };
+
+// The SwiGLU epilogue of one pair's 32 columns c0 .. c0 + 31 (one FP8 group, held by the 4 lanes col + 16 kb as rows 16 j +
+// 4 kb + i of the gate / up accumulators): h = fq8(bf16(w * silu(min(g, L)) * clamp(u, +-L))) (fused.py:284-306).
+__device__ __forceinline__ void swiglu_store(const PrefillArgs& a, const v4f (&gt)[2], const v4f (&up)[2], float wgt, bool store, long long p,
+                                             int c0, int kb) {
+    float h[2][4];
+    float mx = 0.f;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const float gv[4] = {gt[j].x, gt[j].y, gt[j].z, gt[j].w};
+        const float uv[4] = {up[j].x, up[j].y, up[j].z, up[j].w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float gg = gv[i], uu = uv[i];
+            if (a.limit > 0.f) {
+                uu = fminf(fmaxf(uu, -a.limit), a.limit);
+                gg = fminf(gg, a.limit);
+            }
+            float hv = gg * (1.0f / (1.0f + expf(-gg))) * uu;
+            hv = bf16_round(hv * wgt);
+            h[j][i] = hv;
+            mx = fmaxf(mx, fabsf(hv));
+        }
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16));
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    const int ex = fq8_exponent(mx);
+    if (store) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+            *(gmem_u32*)(a.hc + p * a.ldhc + c0 + 16 * j + 4 * kb) = fq8_code4_hw(h[j][0], h[j][1], h[j][2], h[j][3], ex);
+        if (kb == 0) *(gmem_u8*)(a.hs + p * a.ldhs + (c0 >> 5)) = (uint8_t)(ex + 127);
+    }
+}
 
 // Item L of the launch order (group, column blocks) on the 128-pair tile.
 template <int MODE, int TILED>
@@ -807,6 +842,215 @@ __device__ __forceinline__ void prefill_item256(const PrefillArgs& a, const int 
 }
 
 
+// ------------------------------------------------------------------------------------------ light groups
+// Groups of at most 64 pairs on a 256-row x 64-pair tile whose workgroup takes half of a CU: 77 KB of LDS and < 128
+// registers, so two workgroups share the CU and one streams while the other starts, waits at its barrier or runs its
+// epilogue. These groups are bound by the stream of their weights (17 KB a k-step beside <= 8 KB of token rows), not by the
+// matrix pipes; with the one workgroup per CU of the larger tiles every item's start (group tables, token rows, first DMA)
+// and epilogue left the CU's load unit idle, and the weights went through the caches although nothing reads them again.
+// Here an expert's only group reads its weights with non-temporal loads (their E8M0 bytes without: two k-steps' 64 bytes
+// share a cache line; with non-temporal scales w13 at 333 tokens took 777 us), a group with a neighbour of the same expert
+// with cached ones (the neighbour reads them too: Zipf routing at 2048 tokens, w13 1245 us non-temporal, 1105 cached), and
+// the fp32 rows of w2 leave with non-temporal stores (2048 tokens, w2 + combine: 674 -> 643 us).
+// Wave w: row quarter cg = w & 3 as in the tiles above, token blocks 2 u + ph of half ph = w >> 2. One barrier per k-step: it
+// says that every wave's DMA of step k has landed and that every wave has read step k - 1, whose stage then takes
+// step k + 2. Stage: weight slots 16 x 1 KB, their E8M0 bytes, token blocks 4 x 2 KB, the pairs' E8M0 words.
+// Measured against the tiles above (7168 x 1664, 384 experts, top-8, uniform routing, quantiser and dispatch included), w13 /
+// w2 + combine: 48 tokens 611 -> 482 / 292 -> 239 us, 333 tokens 920 -> 747 / 487 -> 430, 1400 tokens 972 -> 877 / 617 ->
+// 568, 2048 tokens 1050 -> 979 / 692 -> 644 (w13 at 333 tokens: 4.87 GB at 6.8 TB/s).
+#define PL_T 64
+#define PL_NS 3
+#define PL_A 0
+#define PL_AS 16384
+#define PL_B 17408
+#define PL_BS (PL_B + 128 * PL_T)
+#define PL_STAGE (PL_BS + 4 * PL_T)
+
+// Column block cb of expert e for the m <= PL_T pairs p0 .. p0 + m - 1. alone: the expert's only pass over these rows.
+template <int MODE, int TILED>
+__device__ __forceinline__ void prefill_pass_light(const PrefillArgs& a, const int e, const int p0, const int m, const int cb, const bool alone) {
+    constexpr int TH = PL_T / 32;   // token blocks per wave
+    extern __shared__ __align__(16) uint8_t smem[];   // PL_NS stages of PL_STAGE bytes
+    __shared__ int s_row[PL_T];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int cg = wave & 3, ph = wave >> 2;
+    const int col = lane & 15, kb = lane >> 4;
+    const int K = a.K, nk = K >> 7, Kh = K >> 1, Ks = K >> 5;
+    const int I = a.N >> 1;
+    auto block_of = [&](int b) {
+        if (MODE == 0) return b < 8 ? (cb * 128 + 16 * b) >> 4 : (I + cb * 128 + 16 * (b - 8)) >> 4;
+        return cb * 16 + b;
+    };
+    const int slot0 = MODE == 0 ? 2 * cg : 4 * cg;   // tile slots slot0 + dslot(j), j = 0..3
+    auto dslot = [](int j) { return MODE == 0 ? (j < 2 ? j : 8 + (j - 2)) : j; };
+    const __amdgpu_buffer_rsrc_t wr = buffer_rsrc(a.W + (long long)e * a.stride_we, (uint32_t)a.stride_we);
+    const __amdgpu_buffer_rsrc_t sr = buffer_rsrc(a.S + (long long)e * a.stride_se, (uint32_t)a.stride_se);
+
+    if (tid < PL_T) {
+        const int p = p0 + (tid < m ? tid : 0);
+        const int r = a.row_of_pair ? a.row_of_pair[p] : p;
+        const int x_rows = (int)(a.xc_bytes / (uint32_t)a.ldx);
+        s_row[tid] = (r >= 0 && r < x_rows) ? r : x_rows;   // x_rows: past both descriptors, reads zeros
+    }
+    float wgt[TH];
+#pragma unroll
+    for (int u = 0; u < TH; ++u) {
+        const int pr = 16 * (2 * u + ph) + col;
+        wgt[u] = MODE == 0 && pr < m ? a.wt_sorted[p0 + pr] : 0.f;
+    }
+    __syncthreads();
+
+    // ---- DMA: wave w loads weight slots 2 w, 2 w + 1 and half w & 1 of token block w >> 1; the slots' E8M0 bytes wave 0
+    // (tiled: 16 B per lane) or waves 0-3 (row-major: 4 slots each, 4 B per lane); the pairs' E8M0 words wave 4
+    auto a_off = [&](int nb) {
+        return TILED ? (uint32_t)(nb * nk * 1024 + col * 64 + kb * 16) : (uint32_t)((nb * 16 + col) * Kh + kb * 16);
+    };
+    const uint32_t a_voff0 = a_off(block_of(2 * wave)), a_voff1 = a_off(block_of(2 * wave + 1));
+    const int a_ks = TILED ? 1024 : 64;
+    const int asb = TILED ? block_of(lane >> 2) : block_of(4 * (wave & 3) + (lane >> 4));
+    const uint32_t as_voff = TILED ? (uint32_t)(asb * nk * 64 + (lane & 3) * 16) : (uint32_t)((asb * 16 + col) * Ks);
+    const int as_ks = TILED ? 64 : 4;
+    const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(a.xc, a.xc_bytes), xsr = buffer_rsrc(a.xs, a.xs_bytes);
+    const int tb_w = wave >> 1;   // the token block this wave loads
+    const uint32_t b_voff = tb_w < PL_T / 16 ? (uint32_t)s_row[16 * (tb_w & (PL_T / 16 - 1)) + col] * (uint32_t)a.ldx + 64 * (wave & 1) + kb * 16 : 0u;
+    const uint32_t bs_voff = (uint32_t)s_row[lane & (PL_T - 1)] * (uint32_t)a.ldxs;
+    const bool ldb = 16 * tb_w < m, lda = TILED ? wave == 0 : wave < 4, ldbs = wave == 4;
+    const int per_step = 2 + (lda ? 1 : 0) + (ldb ? 1 : 0) + (ldbs ? 1 : 0);
+
+    const int lofs = lane * 16;
+    bool tb_on[TH];
+#pragma unroll
+    for (int u = 0; u < TH; ++u) tb_on[u] = 16 * (2 * u + ph) < m;
+    v4f acc[4][TH];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int u = 0; u < TH; ++u) acc[j][u] = v4f{0.f, 0.f, 0.f, 0.f};
+    auto compute = [&](int st) {
+        if (!tb_on[0]) return;   // wave-uniform: no pair in this half
+        const uint8_t* s = smem + st * PL_STAGE;
+        v4i A[4], B0[TH], B1[TH];
+        uint32_t ab[4], bb[TH];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            A[j] = *(const v4i*)(s + PL_A + (slot0 + dslot(j)) * 1024 + lofs);
+            ab[j] = s[PL_AS + (slot0 + dslot(j)) * 64 + col * 4 + kb];
+        }
+#pragma unroll
+        for (int u = 0; u < TH; ++u) {   // a block without pairs reads stale bytes, which no MFMA takes
+            const uint8_t* bt = s + PL_B + (2 * u + ph) * 2048 + lofs;
+            B0[u] = *(const v4i*)bt;
+            B1[u] = *(const v4i*)(bt + 1024);
+            bb[u] = s[PL_BS + (16 * (2 * u + ph) + col) * 4 + kb];
+        }
+        const uint32_t sa = ab[0] | (ab[1] << 8) | (ab[2] << 16) | (ab[3] << 24);
+        uint32_t sb = 0;
+#pragma unroll
+        for (int u = 0; u < TH; ++u) sb |= bb[u] << (8 * u);
+#pragma unroll
+        for (int u = 0; u < TH; ++u) {
+            if (!tb_on[u]) continue;
+            const v8i bv = v8i{B0[u].x, B0[u].y, B0[u].z, B0[u].w, B1[u].x, B1[u].y, B1[u].z, B1[u].w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                acc[j][u] = mfma_fp4w_fp8x_sel(j, u, v8i{A[j].x, A[j].y, A[j].z, A[j].w, 0, 0, 0, 0}, bv, acc[j][u], (int)sa, (int)sb);
+        }
+    };
+    // NT: the weights bypass the caches' replacement order (they are read by this group only)
+    auto kloop = [&](auto ps_c, auto nt_c) __attribute__((always_inline)) {
+        constexpr int PS = decltype(ps_c)::value, PL_AUX = decltype(nt_c)::value ? 2 : 0;
+        uint32_t iao = 0, iso = 0, ixo = 0;
+        auto issue_st = [&](int st) {
+            uint8_t* so = smem + st * PL_STAGE;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void*)(so + PL_A + 2 * wave * 1024), 16, a_voff0, iao, 0, PL_AUX);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void*)(so + PL_A + (2 * wave + 1) * 1024), 16, a_voff1, iao, 0, PL_AUX);
+            if (lda) {
+                if (TILED) __builtin_amdgcn_raw_ptr_buffer_load_lds(sr, (lds_void*)(so + PL_AS), 16, as_voff, iso, 0, 0);
+                else __builtin_amdgcn_raw_ptr_buffer_load_lds(sr, (lds_void*)(so + PL_AS + wave * 256), 4, as_voff, iso, 0, 0);
+            }
+            if (ldb) __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void*)(so + PL_B + wave * 1024), 16, b_voff, ixo, 0, 0);
+            if (ldbs) __builtin_amdgcn_raw_ptr_buffer_load_lds(xsr, (lds_void*)(so + PL_BS), 4, bs_voff, ixo >> 5, 0, 0);
+            iao += a_ks;
+            iso += as_ks;
+            ixo += 128;
+        };
+        // step k in stage st; W: later steps of this wave in flight once its DMA of step k has landed
+        auto step = [&](int st, auto iss_c, auto w_c) __attribute__((always_inline)) {
+            wait_vm_c<PS * decltype(w_c)::value>();
+            __builtin_amdgcn_s_waitcnt((15) | (7 << 4) | (0 << 8) | (3 << 14));   // lgkmcnt(0): own LDS reads of step k - 1 done
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+            if constexpr (decltype(iss_c)::value != 0) issue_st(st == 0 ? PL_NS - 1 : st - 1);
+            compute(st);
+        };
+        issue_st(0);
+        issue_st(1);
+        int st = 0;
+        for (int kk = 0; kk < nk - 2; ++kk) {
+            step(st, IntC<1>{}, IntC<1>{});
+            st = st == PL_NS - 1 ? 0 : st + 1;
+        }
+        step(st, IntC<0>{}, IntC<1>{});
+        st = st == PL_NS - 1 ? 0 : st + 1;
+        step(st, IntC<0>{}, IntC<0>{});
+    };
+    if (alone) {
+        switch (per_step) {
+            case 2: kloop(IntC<2>{}, IntC<1>{}); break;
+            case 3: kloop(IntC<3>{}, IntC<1>{}); break;
+            default: kloop(IntC<4>{}, IntC<1>{}); break;
+        }
+    } else {
+        switch (per_step) {
+            case 2: kloop(IntC<2>{}, IntC<0>{}); break;
+            case 3: kloop(IntC<3>{}, IntC<0>{}); break;
+            default: kloop(IntC<4>{}, IntC<0>{}); break;
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < TH; ++u) {
+        if (!tb_on[u]) continue;
+        const int pr = 16 * (2 * u + ph) + col;
+        if (MODE == 0) {
+            const v4f gt[2] = {acc[0][u], acc[1][u]}, up[2] = {acc[2][u], acc[3][u]};
+            swiglu_store(a, gt, up, wgt[u], pr < m, (long long)p0 + pr, cb * 128 + 32 * cg, kb);
+        } else if (pr < m) {
+            float* o = a.y + (long long)(p0 + pr) * a.ldy + cb * 256 + 64 * cg + 4 * kb;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                gmem_v4f* q = (gmem_v4f*)(o + 16 * j);
+                if (MODE == 2) *q = *q + acc[j][u];
+                else __builtin_nontemporal_store(acc[j][u], q);
+            }
+        }
+    }
+}
+
+// Item L of the launch order (group, column block). A group of more than PL_T pairs takes several passes.
+template <int MODE, int TILED>
+__device__ __forceinline__ void prefill_item_light(const PrefillArgs& a, const int L) {
+    const int jx = L >> 3, gi = jx / a.n_cb;
+    const int g = item_group(a, gi * 8 + (L & 7)), cb = jx - gi * a.n_cb;
+    if (g >= a.G) return;
+    const int e = a.grp_expert[g];
+    if (e < 0 || e >= a.E) return;
+    const int p0 = min(max(a.grp_start[g], 0), a.n_pairs), p1 = p0 + min(min(a.grp_start[g + 1], a.n_pairs) - p0, a.g_max);
+    // no other group of this expert beside this one (a dispatch keeps an expert's groups together)
+    const bool alone = p1 - p0 <= PL_T && (g == 0 || a.grp_expert[g - 1] != e) && (g + 1 >= a.G || a.grp_expert[g + 1] != e);
+    for (int q = p0; q < p1; q += PL_T) {
+        if (q > p0) __syncthreads();   // every wave has read the last pass's rows and operands
+        prefill_pass_light<MODE, TILED>(a, e, q, min(p1 - q, PL_T), cb, alone);
+    }
+}
+
+template <int MODE, int TILED>
+__global__ void __launch_bounds__(PG_THREADS, 4) prefill_gemm_light_kernel(const PrefillArgs a) {
+    if (MODE == 2 && a.run_if && __builtin_amdgcn_readfirstlane(*a.run_if) == 0) return;
+    prefill_item_light<MODE, TILED>(a, (int)blockIdx.x);
+}
+
 // The prefill path's launch: each item takes the 256-pair tile when its group holds more than 128 pairs.
 template <int MODE, int TILED>
 __global__ void __launch_bounds__(PG_THREADS) prefill_gemm_mixed_kernel(const PrefillArgs a) {
@@ -819,15 +1063,22 @@ __global__ void __launch_bounds__(PG_THREADS) prefill_gemm_mixed_kernel(const Pr
     else prefill_item128<MODE, TILED>(a, L);
 }
 
-// mixed: groups of <= 256 pairs (the prefill path's launch); otherwise <= 128 (the 128-pair tile alone)
-static int launch_prefill(PrefillArgs& a, int mode, int tiled, bool mixed, hipStream_t st) {
+// The tile a launch runs its groups on. T_MIXED: groups of <= 256 pairs, by the size of each group; T_128: groups of <= 128
+// pairs; T_LIGHT: tables whose groups hold <= 64 pairs (g_max bounds the pairs of a group that are computed, in passes of 64)
+enum PrefillTile { T_MIXED, T_128, T_LIGHT };
+
+static int launch_prefill(PrefillArgs& a, int mode, int tiled, PrefillTile tile, hipStream_t st) {
+    const bool mixed = tile == T_MIXED, light = tile == T_LIGHT;
     a.g_pad = (a.G + 7) & ~7;
-    a.cbw = (mode == 0 || a.K >= 4096) ? PV_CBW0 : PV_CBW1;   // long k-loops: one column block per workgroup
+    // long k-loops: one column block per workgroup; the light tile too (two: w2 at 2048 tokens 644 -> 659 us, its two
+    // workgroups per CU hide an item's start)
+    a.cbw = (mode == 0 || a.K >= 4096) ? PV_CBW0 : PV_CBW1;
+    if (light) a.cbw = 1;
     a.n_it = (a.n_cb + a.cbw - 1) / a.cbw;
     const long long items = (long long)a.n_it * a.g_pad;   // a multiple of 8
     if (items > 0x7FFFFFFFll) return DSV41_EINVAL;
     const dim3 grid((unsigned)items), block(PG_THREADS);
-    const size_t lds = mixed ? (size_t)max(PV_NS * PV_STAGE, P2_NS * P2_STAGE) : (size_t)PV_NS * PV_STAGE;
+    const size_t lds = light ? (size_t)PL_NS * PL_STAGE : mixed ? (size_t)max(PV_NS * PV_STAGE, P2_NS * P2_STAGE) : (size_t)PV_NS * PV_STAGE;
 #define PV_LAUNCH(K, M, T)                                                                                            \
     do {                                                                                                          \
         const hipError_t err = hipFuncSetAttribute((const void*)K<M, T>, hipFuncAttributeMaxDynamicSharedMemorySize, \
@@ -835,7 +1086,11 @@ static int launch_prefill(PrefillArgs& a, int mode, int tiled, bool mixed, hipSt
         if (err != hipSuccess) return (int)err;                                                                   \
         K<M, T><<<grid, block, lds, st>>>(a);                                                                     \
     } while (0)
-    if (mixed) {
+    if (light) {
+        if (mode == 0) { if (tiled) PV_LAUNCH(prefill_gemm_light_kernel, 0, 1); else PV_LAUNCH(prefill_gemm_light_kernel, 0, 0); }
+        else if (mode == 1) { if (tiled) PV_LAUNCH(prefill_gemm_light_kernel, 1, 1); else PV_LAUNCH(prefill_gemm_light_kernel, 1, 0); }
+        else { if (tiled) PV_LAUNCH(prefill_gemm_light_kernel, 2, 1); else PV_LAUNCH(prefill_gemm_light_kernel, 2, 0); }
+    } else if (mixed) {
         if (mode == 0) { if (tiled) PV_LAUNCH(prefill_gemm_mixed_kernel, 0, 1); else PV_LAUNCH(prefill_gemm_mixed_kernel, 0, 0); }
         else if (mode == 1) { if (tiled) PV_LAUNCH(prefill_gemm_mixed_kernel, 1, 1); else PV_LAUNCH(prefill_gemm_mixed_kernel, 1, 0); }
         else { if (tiled) PV_LAUNCH(prefill_gemm_mixed_kernel, 2, 1); else PV_LAUNCH(prefill_gemm_mixed_kernel, 2, 0); }
@@ -848,10 +1103,10 @@ static int launch_prefill(PrefillArgs& a, int mode, int tiled, bool mixed, hipSt
     return (int)hipGetLastError();
 }
 
-extern "C" int dsv41_prefill_up(const uint8_t* xc, long long ldx, const uint8_t* xs, long long ldxs, int x_rows, const uint8_t* W13, long long stride_we,
+static int prefill_up(PrefillTile tile, const uint8_t* xc, long long ldx, const uint8_t* xs, long long ldxs, int x_rows, const uint8_t* W13, long long stride_we,
                                 const uint8_t* S13, long long stride_se, int tiled, int E, int H, int I, const int* grp_expert,
                                 const int* grp_start, int G, const int* tok_sorted, const float* wt_sorted, float limit, uint8_t* hc,
-                                long long ldhc, uint8_t* hs, long long ldhs, const int* grp_order, void* stream) {
+                      long long ldhc, uint8_t* hs, long long ldhs, const int* grp_order, void* stream) {
     if (!xc || !xs || !W13 || !S13 || !grp_expert || !grp_start || !tok_sorted || !wt_sorted || !hc || !hs) return DSV41_EINVAL;
     if (x_rows < 1 || (long long)x_rows * ldx > 0xFFFFFFFFll || (long long)x_rows * ldxs > 0xFFFFFFFFll) return DSV41_EINVAL;
     if (E < 1 || H < 128 * PG_PF || (H & 127) || I <= 0 || (I & 127) || G < 0 || ldx < H || (ldx & 15) || (((uintptr_t)xc) & 15) || ldxs < H / 32 ||
@@ -864,10 +1119,27 @@ extern "C" int dsv41_prefill_up(const uint8_t* xc, long long ldx, const uint8_t*
     PrefillArgs a{xc, ldx, xs, ldxs, (uint32_t)(x_rows * ldx), (uint32_t)(x_rows * ldxs), W13, stride_we, S13, stride_se, 2 * I, H, E,
                   grp_expert, grp_start, G, tok_sorted, wt_sorted, limit, hc, ldhc, hs, ldhs, nullptr, 0, I / 128, 0, 0x7FFFFFFF};
     a.grp_order = grp_order;
-    return launch_prefill(a, 0, tiled, true, (hipStream_t)stream);
+    a.g_max = P2_T;
+    return launch_prefill(a, 0, tiled, tile, (hipStream_t)stream);
 }
 
-extern "C" int dsv41_prefill_down(const uint8_t* hc, long long ldhc, const uint8_t* hs, long long ldhs, int h_rows, const uint8_t* W2, long long stride_we,
+extern "C" int dsv41_prefill_up(const uint8_t* xc, long long ldx, const uint8_t* xs, long long ldxs, int x_rows, const uint8_t* W13, long long stride_we,
+                                const uint8_t* S13, long long stride_se, int tiled, int E, int H, int I, const int* grp_expert,
+                                const int* grp_start, int G, const int* tok_sorted, const float* wt_sorted, float limit, uint8_t* hc,
+                                long long ldhc, uint8_t* hs, long long ldhs, const int* grp_order, void* stream) {
+    return prefill_up(T_MIXED, xc, ldx, xs, ldxs, x_rows, W13, stride_we, S13, stride_se, tiled, E, H, I, grp_expert, grp_start, G, tok_sorted,
+                      wt_sorted, limit, hc, ldhc, hs, ldhs, grp_order, stream);
+}
+
+extern "C" int dsv41_prefill_up_g64(const uint8_t* xc, long long ldx, const uint8_t* xs, long long ldxs, int x_rows, const uint8_t* W13, long long stride_we,
+                                    const uint8_t* S13, long long stride_se, int tiled, int E, int H, int I, const int* grp_expert,
+                                    const int* grp_start, int G, const int* tok_sorted, const float* wt_sorted, float limit, uint8_t* hc,
+                                    long long ldhc, uint8_t* hs, long long ldhs, const int* grp_order, void* stream) {
+    return prefill_up(T_LIGHT, xc, ldx, xs, ldxs, x_rows, W13, stride_we, S13, stride_se, tiled, E, H, I, grp_expert, grp_start, G, tok_sorted,
+                      wt_sorted, limit, hc, ldhc, hs, ldhs, grp_order, stream);
+}
+
+static int prefill_down(PrefillTile tile, const uint8_t* hc, long long ldhc, const uint8_t* hs, long long ldhs, int h_rows, const uint8_t* W2, long long stride_we,
                                   const uint8_t* S2, long long stride_se, int tiled, int E, int H, int I, const int* grp_expert,
                                   const int* grp_start, int G, float* y2, long long ldy, const int* grp_order, void* stream) {
     if (!hc || !hs || !W2 || !S2 || !grp_expert || !grp_start || !y2) return DSV41_EINVAL;
@@ -882,7 +1154,22 @@ extern "C" int dsv41_prefill_down(const uint8_t* hc, long long ldhc, const uint8
     PrefillArgs a{hc, ldhc, hs, ldhs, (uint32_t)(h_rows * ldhc), (uint32_t)(h_rows * ldhs), W2, stride_we, S2, stride_se, H, I, E,
                   grp_expert, grp_start, G, nullptr, nullptr, 0.f, nullptr, 0, nullptr, 0, y2, ldy, H / 256, 0, h_rows};
     a.grp_order = grp_order;
-    return launch_prefill(a, 1, tiled, true, (hipStream_t)stream);
+    a.g_max = P2_T;
+    return launch_prefill(a, 1, tiled, tile, (hipStream_t)stream);
+}
+
+extern "C" int dsv41_prefill_down(const uint8_t* hc, long long ldhc, const uint8_t* hs, long long ldhs, int h_rows, const uint8_t* W2, long long stride_we,
+                                  const uint8_t* S2, long long stride_se, int tiled, int E, int H, int I, const int* grp_expert,
+                                  const int* grp_start, int G, float* y2, long long ldy, const int* grp_order, void* stream) {
+    return prefill_down(T_MIXED, hc, ldhc, hs, ldhs, h_rows, W2, stride_we, S2, stride_se, tiled, E, H, I, grp_expert, grp_start, G, y2, ldy, grp_order,
+                        stream);
+}
+
+extern "C" int dsv41_prefill_down_g64(const uint8_t* hc, long long ldhc, const uint8_t* hs, long long ldhs, int h_rows, const uint8_t* W2, long long stride_we,
+                                      const uint8_t* S2, long long stride_se, int tiled, int E, int H, int I, const int* grp_expert,
+                                      const int* grp_start, int G, float* y2, long long ldy, const int* grp_order, void* stream) {
+    return prefill_down(T_LIGHT, hc, ldhc, hs, ldhs, h_rows, W2, stride_we, S2, stride_se, tiled, E, H, I, grp_expert, grp_start, G, y2, ldy, grp_order,
+                        stream);
 }
 
 // The groups of a dispatch ordered by pair count, largest first (a counting sort over the counts 0 .. 256 in one
@@ -928,16 +1215,16 @@ static bool lo_term_bad(const uint8_t* xc, const uint8_t* xlc, const uint8_t* xl
            (xlc && xlc == xc);
 }
 
-static int lo_pass(const PrefillArgs& a, const uint8_t* xlc, const uint8_t* xls, const int* lo_flag, int tiled, bool mixed, hipStream_t st) {
+static int lo_pass(const PrefillArgs& a, const uint8_t* xlc, const uint8_t* xls, const int* lo_flag, int tiled, PrefillTile tile, hipStream_t st) {
     if (!xlc) return 0;
     PrefillArgs b = a;
     b.xc = xlc;
     b.xs = xls;
     b.run_if = lo_flag;
-    return launch_prefill(b, 2, tiled, mixed, st);
+    return launch_prefill(b, 2, tiled, tile, st);
 }
 
-extern "C" int dsv41_fp4_grouped_gemm_t128(const uint8_t* xc, long long ldx, const uint8_t* xs, long long ldxs, int x_rows,
+static int grouped_gemm_tile(PrefillTile tile, const uint8_t* xc, long long ldx, const uint8_t* xs, long long ldxs, int x_rows,
                                            const uint8_t* xlc, const uint8_t* xls, const int* lo_flag, const int* row_of_pair,
                                            const uint8_t* W, long long stride_we, const uint8_t* S, long long stride_se, int tiled, int E, int N,
                                            int K, const int* grp_expert, const int* grp_start, int G, int n_pairs, float* y, long long ldy,
@@ -955,8 +1242,27 @@ extern "C" int dsv41_fp4_grouped_gemm_t128(const uint8_t* xc, long long ldx, con
     if (G == 0) return 0;
     PrefillArgs a{xc, ldx, xs, ldxs, (uint32_t)(x_rows * ldx), (uint32_t)(x_rows * ldxs), W, stride_we, S, stride_se, N, K, E,
                   grp_expert, grp_start, G, row_of_pair, nullptr, 0.f, nullptr, 0, nullptr, 0, y, ldy, N / 256, 0, n_pairs};
-    const int rc = launch_prefill(a, 1, tiled, false, (hipStream_t)stream);
-    return rc ? rc : lo_pass(a, xlc, xls, lo_flag, tiled, false, (hipStream_t)stream);
+    a.g_max = PG_T;
+    const int rc = launch_prefill(a, 1, tiled, tile, (hipStream_t)stream);
+    return rc ? rc : lo_pass(a, xlc, xls, lo_flag, tiled, tile, (hipStream_t)stream);
+}
+
+extern "C" int dsv41_fp4_grouped_gemm_t128(const uint8_t* xc, long long ldx, const uint8_t* xs, long long ldxs, int x_rows,
+                                           const uint8_t* xlc, const uint8_t* xls, const int* lo_flag, const int* row_of_pair,
+                                           const uint8_t* W, long long stride_we, const uint8_t* S, long long stride_se, int tiled, int E, int N,
+                                           int K, const int* grp_expert, const int* grp_start, int G, int n_pairs, float* y, long long ldy,
+                                           void* stream) {
+    return grouped_gemm_tile(T_128, xc, ldx, xs, ldxs, x_rows, xlc, xls, lo_flag, row_of_pair, W, stride_we, S, stride_se, tiled, E, N, K, grp_expert,
+                             grp_start, G, n_pairs, y, ldy, stream);
+}
+
+extern "C" int dsv41_fp4_grouped_gemm_t64(const uint8_t* xc, long long ldx, const uint8_t* xs, long long ldxs, int x_rows,
+                                          const uint8_t* xlc, const uint8_t* xls, const int* lo_flag, const int* row_of_pair,
+                                          const uint8_t* W, long long stride_we, const uint8_t* S, long long stride_se, int tiled, int E, int N,
+                                          int K, const int* grp_expert, const int* grp_start, int G, int n_pairs, float* y, long long ldy,
+                                          void* stream) {
+    return grouped_gemm_tile(T_LIGHT, xc, ldx, xs, ldxs, x_rows, xlc, xls, lo_flag, row_of_pair, W, stride_we, S, stride_se, tiled, E, N, K, grp_expert,
+                             grp_start, G, n_pairs, y, ldy, stream);
 }
 
 // out[row_out[p]] (+)= fl(wt[p] * y2[p]) for the pairs of every group g with an expert in [0, E) (its first P2_T pairs,
@@ -1014,7 +1320,7 @@ __global__ void __launch_bounds__(256) scatter_rows_kernel(const float* __restri
 // [row] . deq(W[e_g])^T on the mixed 128 / 256-pair tile kernel (groups of up to 256 pairs), then out[row_out[p]] +=
 // fl(wt[p] * y2[p]) in a second launch (an epilogue of that form inside the tile kernel's k-loop made its compiled loop
 // twice as slow).
-extern "C" int dsv41_fp4_grouped_gemm_scatter(const uint8_t* xc, long long ldx, const uint8_t* xs, long long ldxs, int x_rows,
+static int grouped_gemm_scatter(PrefillTile tile, const uint8_t* xc, long long ldx, const uint8_t* xs, long long ldxs, int x_rows,
                                               const uint8_t* xlc, const uint8_t* xls, const int* lo_flag,
                                               const int* row_of_pair, const uint8_t* W, long long stride_we, const uint8_t* S,
                                               long long stride_se, int tiled, int E, int N, int K, const int* grp_expert, const int* grp_start,
@@ -1037,12 +1343,33 @@ extern "C" int dsv41_fp4_grouped_gemm_scatter(const uint8_t* xc, long long ldx, 
     hipStream_t st = (hipStream_t)stream;
     PrefillArgs a{xc, ldx, xs, ldxs, (uint32_t)(x_rows * ldx), (uint32_t)(x_rows * ldxs), W, stride_we, S, stride_se, N, K, E,
                   grp_expert, grp_start, G, row_of_pair, nullptr, 0.f, nullptr, 0, nullptr, 0, y2, ldy2, N / 256, 0, n_pairs};
-    int rc = launch_prefill(a, 1, tiled, true, st);
-    if (rc == 0) rc = lo_pass(a, xlc, xls, lo_flag, tiled, true, st);
+    a.g_max = P2_T;
+    int rc = launch_prefill(a, 1, tiled, tile, st);
+    if (rc == 0) rc = lo_pass(a, xlc, xls, lo_flag, tiled, tile, st);
     if (rc != 0) return rc;
     const dim3 grid((unsigned)((N + 1023) / 1024), (unsigned)G, P2_T / SCAT_ROWS);
     scatter_rows_kernel<<<grid, 256, 0, st>>>(y2, ldy2, grp_expert, grp_start, E, n_pairs, row_out, wt, distinct, accum, out, ldo, out_rows, N);
     return (int)hipGetLastError();
+}
+
+extern "C" int dsv41_fp4_grouped_gemm_scatter(const uint8_t* xc, long long ldx, const uint8_t* xs, long long ldxs, int x_rows,
+                                              const uint8_t* xlc, const uint8_t* xls, const int* lo_flag, const int* row_of_pair,
+                                              const uint8_t* W, long long stride_we, const uint8_t* S, long long stride_se, int tiled, int E, int N, int K,
+                                              const int* grp_expert, const int* grp_start, int G, int n_pairs, const int* row_out, const float* wt,
+                                              const int* distinct, int accum, float* out, long long ldo, int out_rows, float* y2, long long ldy2,
+                                              void* stream) {
+    return grouped_gemm_scatter(T_MIXED, xc, ldx, xs, ldxs, x_rows, xlc, xls, lo_flag, row_of_pair, W, stride_we, S, stride_se, tiled, E, N, K, grp_expert,
+                                grp_start, G, n_pairs, row_out, wt, distinct, accum, out, ldo, out_rows, y2, ldy2, stream);
+}
+
+extern "C" int dsv41_fp4_grouped_gemm_scatter_g64(const uint8_t* xc, long long ldx, const uint8_t* xs, long long ldxs, int x_rows,
+                                                  const uint8_t* xlc, const uint8_t* xls, const int* lo_flag, const int* row_of_pair,
+                                                  const uint8_t* W, long long stride_we, const uint8_t* S, long long stride_se, int tiled, int E, int N, int K,
+                                                  const int* grp_expert, const int* grp_start, int G, int n_pairs, const int* row_out, const float* wt,
+                                                  const int* distinct, int accum, float* out, long long ldo, int out_rows, float* y2, long long ldy2,
+                                                  void* stream) {
+    return grouped_gemm_scatter(T_LIGHT, xc, ldx, xs, ldxs, x_rows, xlc, xls, lo_flag, row_of_pair, W, stride_we, S, stride_se, tiled, E, N, K, grp_expert,
+                                grp_start, G, n_pairs, row_out, wt, distinct, accum, out, ldo, out_rows, y2, ldy2, stream);
 }
 
 // One workgroup: a bitmap of the output rows in LDS, set by the first n_placed (or n) entries of row_out; an entry whose

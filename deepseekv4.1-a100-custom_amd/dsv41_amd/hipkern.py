@@ -132,6 +132,18 @@ def grouped_gemm_bf16(x: torch.Tensor, permuted: bool, w: torch.Tensor, s: torch
 
 
 T128_MAX = 128   # pairs per group the 128-pair tile kernel computes
+LIGHT_GROUP = 64  # pairs per group of the light tile (two workgroups per CU, csrc/prefill.hip)
+TILE_GROUP = 256  # pairs per group of the larger tiles (128-pair tiles, 256-pair tiles for larger groups)
+LIGHT_PAIRS_PER_EXPERT = 48
+
+
+def tile_group(n_pairs: int, n_experts: int) -> int:
+    """Pairs per group for the tile kernels: LIGHT_GROUP while the pairs average at most LIGHT_PAIRS_PER_EXPERT per expert,
+    else TILE_GROUP. With few pairs per expert the launch is bound by the weight stream, which the light tile runs faster;
+    with more of them an expert's pairs fill several 64-pair groups that each stream its weights. w13 + w2 on either side,
+    larger tiles / light tile (7168 x 1664, 384 experts, top-8): 43 pairs per expert 1742 / 1623 us (uniform routing) and
+    1809 / 1818 (Zipf), 62 pairs per expert 2000 / 2170 and 2130 / 2185."""
+    return LIGHT_GROUP if n_pairs <= LIGHT_PAIRS_PER_EXPERT * n_experts else TILE_GROUP
 
 
 def t128_ok(N: int, K: int, max_tokens: int) -> bool:
@@ -142,16 +154,16 @@ def t128_ok(N: int, K: int, max_tokens: int) -> bool:
 
 def grouped_gemm_t128(xc: torch.Tensor, xs: torch.Tensor, w: torch.Tensor, s: torch.Tensor, grp_expert: torch.Tensor,
                       grp_start: torch.Tensor, row_of_pair: torch.Tensor | None, y: torch.Tensor, n_pairs: int, tiled: bool,
-                      n_cols: int | None = None, lo=None) -> torch.Tensor:
+                      n_cols: int | None = None, lo=None, max_tokens: int = T128_MAX) -> torch.Tensor:
     """y[p, :N] = codes(x)[row_of_pair[p]] . deq(W[e_g])^T for the pairs p of every group (<= 128 pairs each);
-    dsv41_fp4_grouped_gemm_t128."""
+    dsv41_fp4_grouped_gemm_t128, or _t64 (the light tile, the same results) when the groups hold at most 64 pairs."""
     dev = _lib.require_cuda(xc, xs, w, s, grp_expert, grp_start, row_of_pair, y)
     E, N, Kh = w.shape
     N = n_cols if n_cols is not None else N
     K = Kh * 2
     assert w.stride(2) == 1 and w.stride(1) == Kh and s.stride(2) == 1 and s.stride(1) == K // 32
     assert y.dtype == torch.float32 and y.stride(-1) == 1 and y.shape[0] >= n_pairs
-    _lib.call("dsv41_fp4_grouped_gemm_t128", _lib.ptr(xc), xc.stride(0), _lib.ptr(xs), xs.stride(0), xc.shape[0], *_lo_args(lo, xc, xs),
+    _lib.call("dsv41_fp4_grouped_gemm_t64" if max_tokens <= LIGHT_GROUP else "dsv41_fp4_grouped_gemm_t128", _lib.ptr(xc), xc.stride(0), _lib.ptr(xs), xs.stride(0), xc.shape[0], *_lo_args(lo, xc, xs),
               _lib.ptr(row_of_pair),
               _lib.ptr(w), w.stride(0), _lib.ptr(s), s.stride(0), 1 if tiled else 0, E, N, K, _lib.ptr(grp_expert), _lib.ptr(grp_start),
               grp_expert.numel(), n_pairs, _lib.ptr(y), y.stride(0), _lib.stream(dev))
@@ -161,9 +173,10 @@ def grouped_gemm_t128(xc: torch.Tensor, xs: torch.Tensor, w: torch.Tensor, s: to
 def grouped_gemm_scatter(xc: torch.Tensor, xs: torch.Tensor, w: torch.Tensor, s: torch.Tensor, grp_expert: torch.Tensor,
                          grp_start: torch.Tensor, row_of_pair: torch.Tensor | None, row_out: torch.Tensor, wt: torch.Tensor,
                          distinct: torch.Tensor | None, accum: bool, out: torch.Tensor, n_pairs: int, tiled: bool,
-                         n_groups: int | None = None, y2: torch.Tensor | None = None, lo=None) -> torch.Tensor:
+                         n_groups: int | None = None, y2: torch.Tensor | None = None, lo=None,
+                         gmax: int = TILE_GROUP) -> torch.Tensor:
     """out[row_out[p]] += wt[p] * codes(x)[row_of_pair[p]] . deq(W[e_g])^T over the pairs p of the first n_groups
-    groups (<= 256 pairs each; default every table entry); distinct: device int32 scalar, non-zero when no two pairs
+    groups (<= gmax <= 256 pairs each, LIGHT_GROUP taking the light tile; default every table entry); distinct: device int32 scalar, non-zero when no two pairs
     share an output row (then stores when not accum, else read-add-write; otherwise fp32 atomics); y2: fp32
     [n_pairs, N] workspace (allocated when None); dsv41_fp4_grouped_gemm_scatter."""
     dev = _lib.require_cuda(xc, xs, w, s, grp_expert, grp_start, row_of_pair, row_out, wt, distinct, out, y2)
@@ -177,7 +190,7 @@ def grouped_gemm_scatter(xc: torch.Tensor, xs: torch.Tensor, w: torch.Tensor, s:
     if y2 is None:
         y2 = torch.empty(max(n_pairs, 1), N, device=dev, dtype=torch.float32)
     assert y2.dtype == torch.float32 and y2.stride(-1) == 1 and y2.shape[0] >= n_pairs and y2.shape[1] >= N
-    _lib.call("dsv41_fp4_grouped_gemm_scatter", _lib.ptr(xc), xc.stride(0), _lib.ptr(xs), xs.stride(0), xc.shape[0], *_lo_args(lo, xc, xs),
+    _lib.call("dsv41_fp4_grouped_gemm_scatter_g64" if gmax <= LIGHT_GROUP else "dsv41_fp4_grouped_gemm_scatter", _lib.ptr(xc), xc.stride(0), _lib.ptr(xs), xs.stride(0), xc.shape[0], *_lo_args(lo, xc, xs),
               _lib.ptr(row_of_pair),
               _lib.ptr(w), w.stride(0), _lib.ptr(s), s.stride(0), 1 if tiled else 0, E, N, K, _lib.ptr(grp_expert), _lib.ptr(grp_start),
               G, n_pairs, _lib.ptr(row_out), _lib.ptr(wt), _lib.ptr(distinct), 1 if accum else 0, _lib.ptr(out),
@@ -256,8 +269,8 @@ def fp4_gemm_tc(xp: torch.Tensor, w: torch.Tensor, s: torch.Tensor, grp_expert: 
         return out
     xc, xs, lo = _quant_x(xp, True, flag=tile or not lo_in_lds(K, max_tokens))
     if tile:
-        # groups of up to 64 pairs (cukern.FP4_W_MAX): one weight read per group on the 128-pair tile kernel
-        grouped_gemm_t128(xc, xs, w, s, ge, gs, pt, target, n_pairs, FP4_TILED, n_cols=N, lo=lo)
+        # groups of up to 64 pairs (cukern.FP4_W_MAX): one weight read per group on the light or the 128-pair tile kernel
+        grouped_gemm_t128(xc, xs, w, s, ge, gs, pt, target, n_pairs, FP4_TILED, n_cols=N, lo=lo, max_tokens=max_tokens)
         return out
     grouped_gemm_codes(xc, xs, w, s, ge, gs, pt, target, max_tokens, FP4_TILED, shard_start=shard_start,
                        shard_n=shard_n, zero_out=zero_out, n_cols=N, n_pairs=n_pairs, lo=lo)

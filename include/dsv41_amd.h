@@ -176,10 +176,23 @@ int dsv41_prefill_up(const uint8_t* xc, long long ldx, const uint8_t* xs, long l
                      const int* grp_start, int G, const int* tok_sorted, const float* wt_sorted, float limit, uint8_t* hc,
                      long long ldhc, uint8_t* hs, long long ldhs, const int* grp_order, void* stream);
 
+/* dsv41_prefill_up for tables whose groups hold <= 64 pairs (moe_dispatch with gmax <= 64): the same results on a 64-pair tile
+ * whose workgroup takes half of a CU, for few pairs per expert. A larger group is computed in passes of 64 pairs (at
+ * most its first 256). */
+int dsv41_prefill_up_g64(const uint8_t* xc, long long ldx, const uint8_t* xs, long long ldxs, int x_rows, const uint8_t* W13, long long stride_we,
+                     const uint8_t* S13, long long stride_se, int tiled, int E, int H, int I, const int* grp_expert,
+                     const int* grp_start, int G, const int* tok_sorted, const float* wt_sorted, float limit, uint8_t* hc,
+                     long long ldhc, uint8_t* hs, long long ldhs, const int* grp_order, void* stream);
+
 /* Prefill w2: y2[p] = h[p] . deq(W2[e_g])^T (fp32 [P][ldy], sorted pair order) for the same groups; h_rows = P
  * (h_rows * ldhc < 2^32).
  * I % 128 == 0, I >= 384, H % 128 == 0. Replaces the w2 grouped_fp4_gemm of model.py:588. grp_order: as in dsv41_prefill_up. */
 int dsv41_prefill_down(const uint8_t* hc, long long ldhc, const uint8_t* hs, long long ldhs, int h_rows, const uint8_t* W2, long long stride_we,
+                       const uint8_t* S2, long long stride_se, int tiled, int E, int H, int I, const int* grp_expert,
+                       const int* grp_start, int G, float* y2, long long ldy, const int* grp_order, void* stream);
+
+/* dsv41_prefill_down for the tables of dsv41_prefill_up_g64: the same results on the 64-pair tile. */
+int dsv41_prefill_down_g64(const uint8_t* hc, long long ldhc, const uint8_t* hs, long long ldhs, int h_rows, const uint8_t* W2, long long stride_we,
                        const uint8_t* S2, long long stride_se, int tiled, int E, int H, int I, const int* grp_expert,
                        const int* grp_start, int G, float* y2, long long ldy, const int* grp_order, void* stream);
 
@@ -204,6 +217,14 @@ int dsv41_fp4_grouped_gemm_t128(const uint8_t* xc, long long ldx, const uint8_t*
                                 int K, const int* grp_expert, const int* grp_start, int G, int n_pairs, float* y, long long ldy,
                                 void* stream);
 
+/* dsv41_fp4_grouped_gemm_t128 for groups of <= 64 pairs: the same results on the 64-pair tile of dsv41_prefill_up_g64 (a
+ * larger group, of which the first 128 pairs are computed, in passes of 64). */
+int dsv41_fp4_grouped_gemm_t64(const uint8_t* xc, long long ldx, const uint8_t* xs, long long ldxs, int x_rows,
+                                const uint8_t* xlc, const uint8_t* xls, const int* lo_flag, const int* row_of_pair,
+                                const uint8_t* W, long long stride_we, const uint8_t* S, long long stride_se, int tiled, int E, int N,
+                                int K, const int* grp_expert, const int* grp_start, int G, int n_pairs, float* y, long long ldy,
+                                void* stream);
+
 /* moe_kernels.grouped_fp4_gemm with the reference kernel's own epilogue (moe_kernels.py:29-80, 155-200: the tile scaled
  * by the pair weights, then tl.atomic_add into the output rows), on the prefill tile kernels for groups of up to 256
  * pairs (128-pair tiles, 256-pair tiles for groups of more than 128): for each group g (expert in [0, E), pairs clamped
@@ -215,6 +236,14 @@ int dsv41_fp4_grouped_gemm_t128(const uint8_t* xc, long long ldx, const uint8_t*
  * N % 256 == 0, K % 128 == 0, K >= 384, ldo % 4 == 0 and ldy2 % 4 == 0, out and y2 16-byte aligned. xlc / xls /
  * lo_flag: the lo term, as for dsv41_fp4_grouped_gemm_t128 (its pass adds into y2 before the scatter). */
 int dsv41_fp4_grouped_gemm_scatter(const uint8_t* xc, long long ldx, const uint8_t* xs, long long ldxs, int x_rows,
+                                   const uint8_t* xlc, const uint8_t* xls, const int* lo_flag, const int* row_of_pair, const uint8_t* W, long long stride_we, const uint8_t* S,
+                                   long long stride_se, int tiled, int E, int N, int K, const int* grp_expert, const int* grp_start,
+                                   int G, int n_pairs, const int* row_out, const float* wt, const int* distinct, int accum,
+                                   float* out, long long ldo, int out_rows, float* y2, long long ldy2, void* stream);
+
+/* dsv41_fp4_grouped_gemm_scatter for groups of <= 64 pairs, on the 64-pair tile (larger groups, of which the first 256
+ * pairs are computed, in passes of 64). */
+int dsv41_fp4_grouped_gemm_scatter_g64(const uint8_t* xc, long long ldx, const uint8_t* xs, long long ldxs, int x_rows,
                                    const uint8_t* xlc, const uint8_t* xls, const int* lo_flag, const int* row_of_pair, const uint8_t* W, long long stride_we, const uint8_t* S,
                                    long long stride_se, int tiled, int E, int N, int K, const int* grp_expert, const int* grp_start,
                                    int G, int n_pairs, const int* row_out, const float* wt, const int* distinct, int accum,

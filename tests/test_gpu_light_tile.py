@@ -1,0 +1,68 @@
+"""The 64-pair tile of the prefill kernels (dsv41_prefill_up_g64 / _down_g64, dsv41_fp4_grouped_gemm_t64 / _scatter_g64) at
+the edges of its range: group sizes either side of a token block and of the tile (larger groups in passes), experts with one
+group and with several, both weight layouts, the shortest k-loops. Every pair's row is the same sum in the same order as on
+the larger tiles (which are checked against the oracle in test_gpu_moe.py), so the results are equal bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+
+#        expert, pairs: an expert's groups lie together, as a dispatch leaves them
+GROUPS = [(0, 1), (1, 15), (2, 16), (3, 17), (4, 63), (5, 64), (5, 33), (6, 65), (7, 128), (8, 32), (9, 48), (9, 64), (9, 2), (11, 5)]
+
+
+def _setup(H, I, tiled, seed):
+    from dsv41_amd import moe, quant
+    E, T = 12, 77
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    b = lambda *s: torch.randint(0, 256, s, generator=g, dtype=torch.uint8, device=DEV)
+    sc = lambda *s: torch.randint(119, 124, s, generator=g, dtype=torch.uint8, device=DEV)
+    w13, s13, w2, s2 = b(E, 2 * I, H // 2), sc(E, 2 * I, H // 32), b(E, H, I // 2), sc(E, H, I // 32)
+    if tiled:
+        w13, w2, s13, s2 = quant.tile_fp4(w13), quant.tile_fp4(w2), quant.tile_fp4_scales(s13), quant.tile_fp4_scales(s2)
+    P = sum(n for _, n in GROUPS)
+    x = torch.randn(T, H, generator=g, device=DEV).to(torch.bfloat16)
+    i32 = lambda a: torch.tensor(a, dtype=torch.int32, device=DEV)
+    tab = (i32([e for e, _ in GROUPS] + [-1]), i32(np.concatenate([[0], np.cumsum([n for _, n in GROUPS]), [P]])))
+    tok = torch.randint(0, T, (P,), generator=g, device=DEV, dtype=torch.int32)
+    wt = torch.rand(P, generator=g, device=DEV)
+    return moe.ExpertWeights(w13, s13, w2, s2, tiled), x, tab, tok, wt, P
+
+
+@pytest.mark.parametrize("tiled", [True, False])
+@pytest.mark.parametrize("H,I", [(512, 384), (768, 640)])
+def test_light_tile_equals_the_larger_tiles(H, I, tiled):
+    from dsv41_amd import _lib, hipkern, quant
+    print(f"light tile H={H} I={I} tiled={tiled}", flush=True)
+    ex, x, (ge, gs), tok, wt, P = _setup(H, I, tiled, H + I)
+    G, dev = ge.numel(), x.device
+    xc, xs = quant.quant_fp8_e8m0(x)
+    got = {}
+    for suffix in ("", "_g64"):
+        hc = torch.zeros(P, I, dtype=torch.uint8, device=dev)
+        hs = torch.zeros(P, I // 32, dtype=torch.uint8, device=dev)
+        y2 = torch.zeros(P, H, device=dev)
+        _lib.call("dsv41_prefill_up" + suffix, _lib.ptr(xc), xc.stride(0), _lib.ptr(xs), xs.stride(0), x.shape[0], _lib.ptr(ex.w13),
+                  ex.w13.stride(0), _lib.ptr(ex.s13), ex.s13.stride(0), 1 if tiled else 0, ex.E, H, I, _lib.ptr(ge), _lib.ptr(gs), G,
+                  _lib.ptr(tok), _lib.ptr(wt), 10.0, _lib.ptr(hc), hc.stride(0), _lib.ptr(hs), hs.stride(0), None, _lib.stream(dev))
+        _lib.call("dsv41_prefill_down" + suffix, _lib.ptr(hc), hc.stride(0), _lib.ptr(hs), hs.stride(0), P, _lib.ptr(ex.w2), ex.w2.stride(0),
+                  _lib.ptr(ex.s2), ex.s2.stride(0), 1 if tiled else 0, ex.E, H, I, _lib.ptr(ge), _lib.ptr(gs), G, _lib.ptr(y2), y2.stride(0),
+                  None, _lib.stream(dev))
+        # the general grouped GEMM with both FP8 terms of x (the second pass adds), and its scatter form
+        hi, his, lo, los, flag = quant.quant_fp8_split(x)
+        yt = torch.zeros(P, H, device=dev)
+        n = H // 256 * 256
+        hipkern.grouped_gemm_t128(hi, his, ex.w13[:, :n], ex.s13[:, :n], ge, gs, tok, yt, P, tiled, lo=(lo, los, flag),
+                                  max_tokens=64 if suffix else 128)
+        out = torch.zeros(P, n, device=dev)
+        rows = torch.arange(P - 1, -1, -1, dtype=torch.int32, device=dev)
+        one = torch.ones(1, dtype=torch.int32, device=dev)
+        hipkern.grouped_gemm_scatter(hi, his, ex.w13[:, :n], ex.s13[:, :n], ge, gs, tok, rows, wt, one, False, out, P, tiled,
+                                     lo=(lo, los, flag), gmax=64 if suffix else 256)
+        got[suffix] = (hc, hs, y2, yt, out)
+    names = ("h codes", "h scales", "y2", "grouped", "scatter")
+    for name, a, b in zip(names, got[""], got["_g64"]):
+        assert torch.equal(a, b), name
+    assert all(bool(t.any()) for t in got["_g64"])
