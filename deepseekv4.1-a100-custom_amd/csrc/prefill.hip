@@ -60,14 +60,20 @@ __device__ __forceinline__ int item_group(const PrefillArgs& a, int g) {
 // block), which is what bounds the kernel once many tokens share an expert.
 // Every operand moves HBM/L2 -> LDS through the load unit itself (buffer_load ... lds, all through buffer descriptors):
 // no staging registers, PV_NS k-steps (PV_NS x 33 KB) in flight per workgroup. Per k-step, with wave-uniform
-// branches only: wave w loads weight slots 2 w, 2 w + 1 (1 KB each, 16 B per lane) and token block w (two 1 KB
-// halves); the E8M0 bytes of the 16 weight slots (tiled: wave 0, 16 B per lane; row-major: waves 0-3, 4 slots each);
+// branches only: wave w loads weight slots 2 w, 2 w + 1 (1 KB each, 16 B per lane) and token block w (two loads of
+// 1 KB); the E8M0 bytes of the 16 weight slots (tiled: wave 0, 16 B per lane; row-major: waves 0-3, 4 slots each);
 // waves 4-5 the E8M0 words of 64 pairs each.
 // A wave waits for its own loads with vmcnt (they complete in order), then a barrier makes every wave's part
-// visible. The load unit writes lane l's 16 bytes to LDS offset 16 l, and each lane chooses which 16 global
-// bytes it fetches, so the tiles land in MFMA operand order: weight slot s holds, at 16 l, the 16 bytes lane l
-// of the MFMA takes (row l % 16, k chunk l / 16); token block tb holds two 1 KB halves h = 0, 1 with, at 16 l,
-// pair 16 tb + l % 16's k chunk 4 h + l / 16. Every operand read is one contiguous 1 KB ds_read_b128 per wave.
+// visible. The load unit writes lane l's 16 bytes to LDS offset 16 l, and each lane chooses which 16 global bytes it
+// fetches. Consecutive lanes fetch consecutive 16-byte pieces of a row, because the load path takes a quarter of a wave
+// per 64 contiguous bytes it can merge: from L2, 1 KB as whole 64-byte tile rows or 128-byte token rows moves 60 bytes per
+// clock and CU, the same bytes with consecutive lanes on consecutive rows (MFMA operand order) 31 (weight tiles) and 16
+// (token rows). So weight slot s holds the tile's 16 rows of 64 bytes with row R's piece c at position c ^ (R >> 2), and
+// token block tb its 16 pairs' rows of 128 bytes (k chunks 0-7; two loads of 8 rows) with row R's piece c at position
+// c ^ (R >> 1): the pieces are permuted inside the rows only, and the operand reads (lane l of the MFMA takes row l % 16, k
+// chunk l / 16 of the weights, chunks l / 16 and 4 + l / 16 of the pair) of 16 lanes meet all 64 banks once. Measured
+// against operand order: w13 at 8192 tokens (Zipf, 7168 x 1664, 384 experts, top-8, quantiser and dispatch included)
+// 2043 -> 1876 us, w2 + combine 1612 -> 1561, w13 at 2048 tokens 972 -> 920.
 // Wave w computes 4 row blocks (MODE 0: gate slots 2 cg, 2 cg + 1 and their up slots, cg = w & 3, one FP8 group
 // of 32 columns) for the 64 pairs of half w >> 2: 4 x 4 accumulators, 192 B of LDS reads per lane per k-step
 // for 16 MFMAs. The operands of step k + 1 are read while the MFMAs of step k run; stage k is refilled with
@@ -204,10 +210,11 @@ __device__ __forceinline__ void prefill_item128(const PrefillArgs& a, const int 
     }
     __syncthreads();
 
-    // ---- DMA descriptors (MFMA A layout: lane l takes row l % 16, k chunk l / 16)
+    // ---- DMA descriptors (weight slots: lane l fetches a piece of row l / 4)
     const int nbw0 = block_of(2 * wave, cb0), nbw1 = block_of(2 * wave + 1, cb0);
+    const int a_pc = ((lane & 3) ^ (lane >> 4)) * 16;   // this lane's piece of row lane / 4
     auto a_off = [&](int nb) {
-        return TILED ? (uint32_t)(nb * nk * 1024 + col * 64 + kb * 16) : (uint32_t)((nb * 16 + col) * Kh + kb * 16);
+        return TILED ? (uint32_t)(nb * nk * 1024 + (lane >> 2) * 64 + a_pc) : (uint32_t)((nb * 16 + (lane >> 2)) * Kh + a_pc);
     };
     const uint32_t a_voff0 = a_off(nbw0), a_voff1 = a_off(nbw1);
     const int a_ks = TILED ? 1024 : 64;
@@ -219,11 +226,12 @@ __device__ __forceinline__ void prefill_item128(const PrefillArgs& a, const int 
     const uint32_t as_voff = TILED ? (uint32_t)(asb * nk * 64 + (lane & 3) * 16) : (uint32_t)((asb * 16 + asr) * Ks);
     const int as_ks = TILED ? 64 : 4;
     const uint32_t as_cs = TILED ? (uint32_t)(PV_DNB * nk * 64) : (uint32_t)(PV_DNB * 16 * Ks);
-    // MFMA B layout of token block `wave`: half h, lane l takes pair 16 wave + l % 16, k chunk 4 h + l / 16
+    // token block `wave`: two loads of 8 rows, lane l fetches a piece of row l / 8
     // activation rows through buffer descriptors too: reads past x_rows return 0, and with no FLAT-encoded load in
     // flight the compiler's waits on the LDS operand reads stay partial instead of draining all of them
     const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(a.xc, a.xc_bytes), xsr = buffer_rsrc(a.xs, a.xs_bytes);
-    const uint32_t b0off = (uint32_t)s_row[16 * wave + col] * (uint32_t)a.ldx + kb * 16;
+    const uint32_t b0off = (uint32_t)s_row[16 * wave + (lane >> 3)] * (uint32_t)a.ldx + ((lane & 7) ^ (lane >> 4)) * 16;
+    const uint32_t b1off = (uint32_t)s_row[16 * wave + 8 + (lane >> 3)] * (uint32_t)a.ldx + ((lane & 7) ^ (4 + (lane >> 4))) * 16;
     const uint32_t bsoff = (uint32_t)s_row[(64 * (wave & 1) + lane) & (PG_T - 1)] * (uint32_t)a.ldxs;
     const bool ldb = 16 * wave < m;   // wave-uniform: the token block holds pairs of the group
     const bool lda = TILED ? wave == 0 : wave < 4, ldbs = (wave == 4 || wave == 5) && 64 * (wave & 1) < m;
@@ -242,14 +250,15 @@ __device__ __forceinline__ void prefill_item128(const PrefillArgs& a, const int 
         }
         if (decltype(full_c)::value || ldb) {
             __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void*)(so + PV_B + wave * 2048), 16, b0off, (uint32_t)(kc * 128), 0, 0);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void*)(so + PV_B + wave * 2048 + 1024), 16, b0off + 64, (uint32_t)(kc * 128), 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void*)(so + PV_B + wave * 2048 + 1024), 16, b1off, (uint32_t)(kc * 128), 0, 0);
         }
         if (ldbs)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(xsr, (lds_void*)(so + PV_BS + (wave - 4) * 256), 4, bsoff, (uint32_t)(kc * 4), 0, 0);
     };
 
     // ---- operand registers (double-buffered) and their LDS reads
-    const int lofs = lane * 16;
+    const int lofs = col * 64 + ((kb ^ (col >> 2)) * 16);                                                     // weight slot
+    const int bofs0 = col * 128 + ((kb ^ (col >> 1)) * 16), bofs1 = col * 128 + (((4 + kb) ^ (col >> 1)) * 16);   // token block, k half 0 / 1
     bool tb_on[4];   // token blocks holding pairs (wave-uniform)
 #pragma unroll
     for (int u = 0; u < 4; ++u) tb_on[u] = 64 * ph + 16 * u < m;
@@ -270,9 +279,9 @@ __device__ __forceinline__ void prefill_item128(const PrefillArgs& a, const int 
             }
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                const uint8_t* bt = st + PV_B + (4 * ph + u) * 2048 + lofs;
-                OB0[r][u] = *(const v4i*)bt;
-                OB1[r][u] = *(const v4i*)(bt + 1024);
+                const uint8_t* bt = st + PV_B + (4 * ph + u) * 2048;
+                OB0[r][u] = *(const v4i*)(bt + bofs0);
+                OB1[r][u] = *(const v4i*)(bt + bofs1);
                 bb[u] = st[PV_BS + (64 * ph + 16 * u + col) * 4 + kb];
             }
             OSA[r] = ab[0] | (ab[1] << 8) | (ab[2] << 16) | (ab[3] << 24);
@@ -616,11 +625,12 @@ __device__ __forceinline__ void prefill_item256(const PrefillArgs& a, const int 
     }
     __syncthreads();
 
-    // ---- DMA descriptors: weight slots 2 w, 2 w + 1; token blocks 2 w, 2 w + 1 (two 1 KB halves each); weight scales
+    // ---- DMA descriptors: weight slots 2 w, 2 w + 1; token blocks 2 w, 2 w + 1 (two loads of 8 rows each); weight scales
     // (tiled: wave 0, 16 B per lane; row-major: waves 0-3, 4 slots each); the pairs' E8M0 words (waves 4-7, 64 each)
     const int nbw0 = block_of(2 * wave, cb0), nbw1 = block_of(2 * wave + 1, cb0);
+    const int a_pc = ((lane & 3) ^ (lane >> 4)) * 16;   // this lane's piece of row lane / 4
     auto a_off = [&](int nb) {
-        return TILED ? (uint32_t)(nb * nk * 1024 + col * 64 + kb * 16) : (uint32_t)((nb * 16 + col) * Kh + kb * 16);
+        return TILED ? (uint32_t)(nb * nk * 1024 + (lane >> 2) * 64 + a_pc) : (uint32_t)((nb * 16 + (lane >> 2)) * Kh + a_pc);
     };
     const uint32_t a_voff0 = a_off(nbw0), a_voff1 = a_off(nbw1);
     const int a_ks = TILED ? 1024 : 64;
@@ -630,14 +640,17 @@ __device__ __forceinline__ void prefill_item256(const PrefillArgs& a, const int 
     const int as_ks = TILED ? 64 : 4;
     const uint32_t as_cs = TILED ? (uint32_t)(PV_DNB * nk * 64) : (uint32_t)(PV_DNB * 16 * Ks);
     const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(a.xc, a.xc_bytes), xsr = buffer_rsrc(a.xs, a.xs_bytes);
-    const uint32_t b0off = (uint32_t)s_row[32 * wave + col] * (uint32_t)a.ldx + kb * 16;
-    const uint32_t b1off = (uint32_t)s_row[32 * wave + 16 + col] * (uint32_t)a.ldx + kb * 16;
+    uint32_t boff[4];   // rows 32 wave + 8 i ..
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        boff[i] = (uint32_t)s_row[32 * wave + 8 * i + (lane >> 3)] * (uint32_t)a.ldx + ((lane & 7) ^ (4 * (i & 1) + (lane >> 4))) * 16;
     const uint32_t bsoff = (uint32_t)s_row[(64 * (wave & 3) + lane) & (P2_T - 1)] * (uint32_t)a.ldxs;
     const bool ldb0 = 32 * wave < m, ldb1 = 32 * wave + 16 < m;   // wave-uniform: the token block holds pairs
     const bool lda = TILED ? wave == 0 : wave < 4, ldbs = wave >= 4 && 64 * (wave - 4) < m;
     const int per_step = 2 + (lda ? 1 : 0) + (ldb0 ? 2 : 0) + (ldb1 ? 2 : 0) + (ldbs ? 1 : 0);
 
-    const int lofs = lane * 16;
+    const int lofs = col * 64 + ((kb ^ (col >> 2)) * 16);                                                     // weight slot
+    const int bofs0 = col * 128 + ((kb ^ (col >> 1)) * 16), bofs1 = col * 128 + (((4 + kb) ^ (col >> 1)) * 16);   // token block, k half 0 / 1
     bool tb_on[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) tb_on[u] = 16 * (2 * u + ph) < m;
@@ -645,7 +658,7 @@ __device__ __forceinline__ void prefill_item256(const PrefillArgs& a, const int 
     v4i OA[4], OB0[8], OB1[8];
     uint32_t OSA, OSB[2];
     // per-lane LDS offsets within a stage: weight slots relative to slot_of[0], token blocks of this half, scales
-    const uint32_t lofs_a = (uint32_t)(P2_A + slot_of[0] * 1024 + lofs), lofs_b = (uint32_t)(P2_B + ph * 2048 + lofs);
+    const uint32_t lofs_a = (uint32_t)(P2_A + slot_of[0] * 1024 + lofs), lofs_b = (uint32_t)(P2_B + ph * 2048 + bofs0), lofs_b1 = (uint32_t)(P2_B + ph * 2048 + bofs1);
     const uint32_t lofs_as = (uint32_t)(P2_AS + slot_of[0] * 64 + col * 4 + kb), lofs_bs = (uint32_t)(P2_BS + 16 * ph * 4 + col * 4 + kb);
     // Every read of a step is issued before any of them is used: the token blocks unconditionally (a block without
     // pairs reads stale bytes of its slot, which no MFMA takes) and each E8M0 byte into a register of its own, packed
@@ -653,7 +666,7 @@ __device__ __forceinline__ void prefill_item256(const PrefillArgs& a, const int 
     // eight serial round trips per step, the longest part of the step.)
     auto read_ops = [&](int st) {
         const uint32_t so = (uint32_t)st * P2_STAGE;
-        const uint32_t oa = lofs_a + so, ob = lofs_b + so, osa = lofs_as + so, osb = lofs_bs + so;
+        const uint32_t oa = lofs_a + so, ob = lofs_b + so, ob1 = lofs_b1 + so, osa = lofs_as + so, osb = lofs_bs + so;
         uint32_t ab[4], bb[8];
         if (any_on) {   // wave-uniform: a wave whose half of the group is empty reads and computes nothing
 #pragma unroll
@@ -665,7 +678,7 @@ __device__ __forceinline__ void prefill_item256(const PrefillArgs& a, const int 
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
                 OB0[u] = *(const v4i*)(smem + ob + u * 4096);
-                OB1[u] = *(const v4i*)(smem + ob + u * 4096 + 1024);
+                OB1[u] = *(const v4i*)(smem + ob1 + u * 4096);
                 bb[u] = smem[osb + u * 128];
             }
             OSA = ab[0] | (ab[1] << 8) | (ab[2] << 16) | (ab[3] << 24);
@@ -766,12 +779,12 @@ __device__ __forceinline__ void prefill_item256(const PrefillArgs& a, const int 
                 else __builtin_amdgcn_raw_ptr_buffer_load_lds(sr, (lds_void*)(so + P2_AS + wave * 256), 4, as_voff, iso, 0, 0);
             }
             if (ldb0) {
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void*)(so + P2_B + 2 * wave * 2048), 16, b0off, ixo, 0, 0);
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void*)(so + P2_B + 2 * wave * 2048 + 1024), 16, b0off + 64, ixo, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void*)(so + P2_B + 2 * wave * 2048), 16, boff[0], ixo, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void*)(so + P2_B + 2 * wave * 2048 + 1024), 16, boff[1], ixo, 0, 0);
             }
             if (ldb1) {
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void*)(so + P2_B + (2 * wave + 1) * 2048), 16, b1off, ixo, 0, 0);
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void*)(so + P2_B + (2 * wave + 1) * 2048 + 1024), 16, b1off + 64, ixo, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void*)(so + P2_B + (2 * wave + 1) * 2048), 16, boff[2], ixo, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void*)(so + P2_B + (2 * wave + 1) * 2048 + 1024), 16, boff[3], ixo, 0, 0);
             }
             if (ldbs)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(xsr, (lds_void*)(so + P2_BS + (wave - 4) * 256), 4, bsoff, ixo >> 5, 0, 0);
@@ -902,10 +915,11 @@ __device__ __forceinline__ void prefill_pass_light(const PrefillArgs& a, const i
     }
     __syncthreads();
 
-    // ---- DMA: wave w loads weight slots 2 w, 2 w + 1 and half w & 1 of token block w >> 1; the slots' E8M0 bytes wave 0
+    // ---- DMA: wave w loads weight slots 2 w, 2 w + 1 and 8 rows (half w & 1) of token block w >> 1; the slots' E8M0 bytes wave 0
     // (tiled: 16 B per lane) or waves 0-3 (row-major: 4 slots each, 4 B per lane); the pairs' E8M0 words wave 4
+    const int a_pc = ((lane & 3) ^ (lane >> 4)) * 16;   // this lane's piece of row lane / 4
     auto a_off = [&](int nb) {
-        return TILED ? (uint32_t)(nb * nk * 1024 + col * 64 + kb * 16) : (uint32_t)((nb * 16 + col) * Kh + kb * 16);
+        return TILED ? (uint32_t)(nb * nk * 1024 + (lane >> 2) * 64 + a_pc) : (uint32_t)((nb * 16 + (lane >> 2)) * Kh + a_pc);
     };
     const uint32_t a_voff0 = a_off(block_of(2 * wave)), a_voff1 = a_off(block_of(2 * wave + 1));
     const int a_ks = TILED ? 1024 : 64;
@@ -914,12 +928,14 @@ __device__ __forceinline__ void prefill_pass_light(const PrefillArgs& a, const i
     const int as_ks = TILED ? 64 : 4;
     const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(a.xc, a.xc_bytes), xsr = buffer_rsrc(a.xs, a.xs_bytes);
     const int tb_w = wave >> 1;   // the token block this wave loads
-    const uint32_t b_voff = tb_w < PL_T / 16 ? (uint32_t)s_row[16 * (tb_w & (PL_T / 16 - 1)) + col] * (uint32_t)a.ldx + 64 * (wave & 1) + kb * 16 : 0u;
+    const uint32_t b_voff = tb_w < PL_T / 16 ? (uint32_t)s_row[16 * (tb_w & (PL_T / 16 - 1)) + 8 * (wave & 1) + (lane >> 3)] * (uint32_t)a.ldx +
+                                                     ((lane & 7) ^ (4 * (wave & 1) + (lane >> 4))) * 16 : 0u;
     const uint32_t bs_voff = (uint32_t)s_row[lane & (PL_T - 1)] * (uint32_t)a.ldxs;
     const bool ldb = 16 * tb_w < m, lda = TILED ? wave == 0 : wave < 4, ldbs = wave == 4;
     const int per_step = 2 + (lda ? 1 : 0) + (ldb ? 1 : 0) + (ldbs ? 1 : 0);
 
-    const int lofs = lane * 16;
+    const int lofs = col * 64 + ((kb ^ (col >> 2)) * 16);                                                     // weight slot
+    const int bofs0 = col * 128 + ((kb ^ (col >> 1)) * 16), bofs1 = col * 128 + (((4 + kb) ^ (col >> 1)) * 16);   // token block, k half 0 / 1
     bool tb_on[TH];
 #pragma unroll
     for (int u = 0; u < TH; ++u) tb_on[u] = 16 * (2 * u + ph) < m;
@@ -940,9 +956,9 @@ __device__ __forceinline__ void prefill_pass_light(const PrefillArgs& a, const i
         }
 #pragma unroll
         for (int u = 0; u < TH; ++u) {   // a block without pairs reads stale bytes, which no MFMA takes
-            const uint8_t* bt = s + PL_B + (2 * u + ph) * 2048 + lofs;
-            B0[u] = *(const v4i*)bt;
-            B1[u] = *(const v4i*)(bt + 1024);
+            const uint8_t* bt = s + PL_B + (2 * u + ph) * 2048;
+            B0[u] = *(const v4i*)(bt + bofs0);
+            B1[u] = *(const v4i*)(bt + bofs1);
             bb[u] = s[PL_BS + (16 * (2 * u + ph) + col) * 4 + kb];
         }
         const uint32_t sa = ab[0] | (ab[1] << 8) | (ab[2] << 16) | (ab[3] << 24);
