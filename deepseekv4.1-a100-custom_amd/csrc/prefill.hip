@@ -358,7 +358,7 @@ __device__ __forceinline__ void prefill_item128(const PrefillArgs& a, const int 
                     for (int j = 0; j < 4; ++j) {
                         gmem_v4f* q = (gmem_v4f*)(o + 16 * j);
                         if (MODE == 2) *q = *q + acc[j][u];   // the lo term's pass adds to the hi term's rows
-                        else *q = acc[j][u];
+                        else __builtin_nontemporal_store(acc[j][u], q);
                     }
                 }
             }
@@ -514,7 +514,8 @@ __global__ void __launch_bounds__(PG_THREADS) prefill_gemm_lds_kernel(const Pref
 }
 
 // y[t][n] = bf16(sum_j y2[inv[t * topk + j]][n] (+ ys[t][n])), j ascending (model.py:589-591: view(n, k, dim).sum(1)
-// then + shared, fp32); optional fp32 y32. One thread per 4 consecutive n.
+// then + shared, fp32); optional fp32 y32. One thread per 4 consecutive n. Bound by the read of y2, which nothing reads
+// again: non-temporal loads (w2 + combine at 2048 / 8192 tokens, 7168 x 1664, top-8: 630 -> 598 / 1570 -> 1533 us).
 __global__ void __launch_bounds__(256) combine_pairs_kernel(const float* __restrict__ y2, long long ldy2, const int* __restrict__ inv,
                                                             int topk, int T, int N, const uint16_t* __restrict__ ys, long long ldys,
                                                             uint16_t* __restrict__ out, long long ldo, float* __restrict__ y32, long long ld32) {
@@ -531,7 +532,7 @@ __global__ void __launch_bounds__(256) combine_pairs_kernel(const float* __restr
         for (int j = 0; j < 8; ++j) r[j] = j < topk ? inv[t * topk + j] : -1;
         v4f v[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = r[j] >= 0 ? *(const v4f*)(y2 + (long long)r[j] * ldy2 + n) : v4f{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < 8; ++j) v[j] = r[j] >= 0 ? __builtin_nontemporal_load((const v4f*)(y2 + (long long)r[j] * ldy2 + n)) : v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int j = 0; j < 8; ++j)
             if (r[j] >= 0) s += v[j];
@@ -751,7 +752,7 @@ __device__ __forceinline__ void prefill_item256(const PrefillArgs& a, const int 
                     for (int j = 0; j < 4; ++j) {
                         gmem_v4f* q = (gmem_v4f*)(o + 16 * j);
                         if (MODE == 2) *q = *q + acc[j][u];   // the lo term's pass adds to the hi term's rows
-                        else *q = acc[j][u];
+                        else __builtin_nontemporal_store(acc[j][u], q);
                     }
                 }
             }
