@@ -341,6 +341,46 @@ def fp8_gemm_tc(x: torch.Tensor, w8: torch.Tensor, s8: torch.Tensor, group_cols:
     return y if out_dtype == torch.float32 else y.to(out_dtype)
 
 
+def fp8_rows_plan(M: int, N: int, K: int):
+    """(activation rows per tile, K ranges) with which dsv41_fp8_gemm_rows multiplies M > 64 rows, or None where dequantising
+    the weights and the library GEMM are faster.
+    Tiles of 64 rows while they fit the CUs once, K split until about 256 workgroups (ranges of at least 1024 k); else tiles
+    of 128 up to 512 rows, and beyond them up to 1024 rows while one such tile per CU covers the product. us, dequantised +
+    library / tiles: 5120 x 8192 at 100 rows 72 / 33, 333 86 / 53, 700 106 / 77, 1400 143 / 132; 32768 x 1280 at 333 77 / 56,
+    700 104 / 102, 1400 147 / 186; 1280 x 5120 at 333 29 / 24, 700 35 / 34; 3328 x 7168 at 333 66 / 47, 700 80 / 68, 1400
+    99 / 105; 7168 x 1664 at 333 35 / 24, 700 40 / 40."""
+    if K % 64 or N % 8 or M > 1024:
+        return None
+    tn = (N + 127) // 128
+    t64, t128 = tn * ((M + 63) // 64), tn * ((M + 127) // 128)
+    if t64 <= 256:
+        tile, splits = 64, max(1, min(256 // t64, K // 1024, 8))
+    elif M <= 512 or t128 <= 256:
+        tile, splits = 128, 1
+    else:
+        return None
+    # a range's scale bytes fit the kernel's 512
+    return (tile, splits) if 2 * (-(-(K // 64) // splits)) <= 512 else None
+
+
+def fp8_gemm_rows(x: torch.Tensor, w8: torch.Tensor, s8: torch.Tensor, tiled: bool, plan) -> torch.Tensor:
+    """bf16 [M, N] = x . deq(w8)^T for M rows of contiguous bf16 x with plan = fp8_rows_plan(M, N, K); the values of
+    fp8_gemm_tc up to the order of the fp32 sums. dsv41_fp8_gemm_rows."""
+    dev = _lib.require_cuda(x, w8, s8)
+    M, K = x.shape
+    N = w8.shape[0]
+    tile, splits = plan
+    assert x.dtype == torch.bfloat16 and x.is_contiguous() and w8.is_contiguous() and w8.dtype == torch.uint8 and s8.dtype == torch.uint8
+    assert x.data_ptr() % 16 == 0 and w8.data_ptr() % 16 == 0
+    if s8.dim() != 2 or s8.shape[0] < (N + 31) // 32 or s8.shape[1] < K // 32 or s8.stride(1) != 1 or w8.shape[1] != K:
+        raise ValueError(f"fp8 operands: {tuple(w8.shape)} weights with {tuple(s8.shape)} scales for K = {K}")
+    y = torch.empty(M, N, device=dev, dtype=torch.bfloat16)
+    part = torch.empty(splits * M * N, device=dev, dtype=torch.float32) if splits > 1 else None
+    _lib.call("dsv41_fp8_gemm_rows", _lib.ptr(w8), K, 1 if tiled else 0, _lib.ptr(s8), s8.stride(0), N, K, _lib.ptr(x), K, M, None, 0,
+              _lib.ptr(y), N, tile, splits, _lib.ptr(part), splits * M * N if splits > 1 else 0, _lib.stream(dev))
+    return y
+
+
 def fp8_gemv(x: torch.Tensor, w_fp8: torch.Tensor, s_u8: torch.Tensor) -> torch.Tensor:
     """x: bf16 [M, K]; w_fp8: float8_e4m3fn / uint8 [N, K] row-major (any N); s_u8: uint8 [ceil(N/32), K/32] (E8M0).
     fp32 [M, N] (cukern.py:78-93; the reference takes M == 1, this takes M <= 64). K % 32 == 0: a K that is not a

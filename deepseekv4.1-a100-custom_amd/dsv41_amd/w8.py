@@ -4,9 +4,9 @@ model.linear_fp8 (model.py:55-58).
 
 Up to 64 rows run through dsv41_fp8_gemm (csrc/dense_fp8.hip): the weights are streamed once as FP8 (half the bytes
 of bf16), decoded in registers to bf16 MFMA operands with their block scale and accumulated in fp32, which gives the
-same numbers as the bf16 product up to the order of the fp32 additions (w8.py:1-7). More rows (prefill) dequantize
-to a bf16 matrix, or use the kept bf16 copy, and call the library GEMM, as the reference does past its kernels'
-row limits (w8.py:102-113).
+same numbers as the bf16 product up to the order of the fp32 additions (w8.py:1-7). A few hundred rows take the same
+arithmetic in tiles (dsv41_fp8_gemm_rows); more rows (prefill) dequantize to a bf16 matrix, or use the kept bf16 copy,
+and call the library GEMM, as the reference does past its kernels' row limits (w8.py:102-113).
 
 Stored byte order: the MFMA fragments of the HIP kernel take k in natural order, so permute_k is the identity
 (PERM_K is kept for drop-in code that indexes it). tile() is this build's 1 KiB tile order
@@ -115,18 +115,35 @@ class W8:
         return W8(torch.cat([w.w8 for w in ws], dim=0), torch.cat([w.s8 for w in ws], dim=0), permuted=True, tiled=ws[0].tiled)
 
 
+def _tiles_ok(x: torch.Tensor, w: "W8") -> bool:
+    """Whether x . w^T can take the FP8 tiles: GPU tensors of 16-byte rows whose bytes 32-bit offsets reach, and nothing that
+    watches the call (gradients, forward-mode, vmap, tracing, autocast, tensor subclasses): those keep F.linear."""
+    if type(x) is not torch.Tensor or torch.compiler.is_compiling() or torch._C._functorch.is_functorch_wrapped_tensor(x):
+        return False
+    if (torch.is_grad_enabled() and x.requires_grad) or torch.autograd.forward_ad._current_level >= 0 or torch.is_autocast_enabled():
+        return False
+    return (x.device == w.w8.device and x.is_cuda and x.shape[1] == w.shape[1] and (x.data_ptr() % 16 == 0 or not x.is_contiguous())
+            and w.w8.data_ptr() % 16 == 0 and x.numel() * 2 < 1 << 31 and 128 * w.shape[1] < 1 << 31)
+
+
 def linear_w(x: torch.Tensor, w) -> torch.Tensor:
     """y = x . w^T with bf16 activations and a bf16 result, for w a plain bf16 tensor (library GEMM) or a W8
-    (w8.py:102-113): up to MAX_TC_ROWS rows the FP8 launch reads the E4M3 bytes directly, beyond that (or from
-    BF16_ROWS rows with a kept copy) the library GEMM runs on the dequantised weights."""
+    (w8.py:102-113): up to MAX_TC_ROWS rows the FP8 launch reads the E4M3 bytes directly, and for some hundred rows more its
+    tiled form does (hipkern.fp8_rows_plan); beyond that (or from BF16_ROWS rows with a kept copy) the library GEMM runs on
+    the dequantised weights."""
     if not isinstance(w, W8):
         return F.linear(x, w)
     lead = x.shape[:-1]
     x2 = x.reshape(-1, x.shape[-1])
     if x2.shape[0] <= MAX_TC_ROWS and (w.bf16w is None or x2.shape[0] < BF16_ROWS):
         y = hipkern.fp8_gemm_tc(x2.contiguous().to(torch.bfloat16), w.w8, w.s8, tiled=w.tiled)
+        return y.view(*lead, w.shape[0])
+    xb = x2.to(torch.bfloat16)
+    plan = hipkern.fp8_rows_plan(x2.shape[0], *w.shape) if w.bf16w is None and _tiles_ok(xb, w) else None
+    if plan is not None:
+        y = hipkern.fp8_gemm_rows(xb.contiguous(), w.w8, w.s8, w.tiled, plan)
     else:
-        y = F.linear(x2.to(torch.bfloat16), w.bf16())
+        y = F.linear(xb, w.bf16())
     return y.view(*lead, w.shape[0])
 
 

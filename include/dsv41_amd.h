@@ -318,6 +318,15 @@ int dsv41_fp8_gemm(const uint8_t* W, long long ldw, int tiled, const uint8_t* S,
                    const uint16_t* x, long long ldx, int M, int group_cols, float* out, long long ldo,
                    uint16_t* outb, long long ldob, void* stream);
 
+/* dsv41_fp8_gemm for any number of rows (no column groups): 128 weight rows x `tile` (64 or 128) activation rows per workgroup,
+ * K in `splits` ranges (at most K / 64; a range holds at most 256 chunks of 64 k). splits > 1: part is an fp32 workspace of at
+ * least splits * M * N floats (16-byte aligned, N % 4 == 0), whose ranges a second launch adds in order. x and W 16-byte
+ * aligned, ldx % 8 == 0, row-major ldw % 16 == 0, M * ldx * 2 < 2^31. Replaces the dequantisation + library GEMM of
+ * w8.linear_w past the 64 rows of dsv41_fp8_gemm (w8.py:102-113). */
+int dsv41_fp8_gemm_rows(const uint8_t* W, long long ldw, int tiled, const uint8_t* S, long long lds, int N, int K,
+                        const uint16_t* x, long long ldx, int M, float* out, long long ldo, uint16_t* outb, long long ldob,
+                        int tile, int splits, float* part, long long part_floats, void* stream);
+
 /* W8.bf16 / quant.dequant_fp8_block (w8.py:78-82, quant.py:90-95): out bf16 [N][ldo] = bf16(e4m3(W) * 2^(S - 127)),
  * the fp32 product rounded to bf16 (bit-exact). W in either layout of dsv41_fp8_gemm (tiled needs K % 64 == 0);
  * K % 16 == 0. */
