@@ -48,62 +48,66 @@ extern "C" int dsv41_gate_topk(const float* scores, long long lds, const float* 
 #define DISP_WAVES (DISP_THREADS / WAVE)
 #define DISP_MAX_E 512
 
-// exclusive scan of v over the block's threads (fixed order); the block total lands in *total
-__device__ __forceinline__ int block_exclusive_scan(int v, int* s_scan, int* total) {
-    const int tid = threadIdx.x;
-    s_scan[tid] = v;
-    __syncthreads();
-    for (int o = 1; o < DISP_THREADS; o <<= 1) {   // Hillis-Steele inclusive scan
-        const int t = tid >= o ? s_scan[tid - o] : 0;
-        __syncthreads();
-        s_scan[tid] += t;
-        __syncthreads();
+// exclusive scans of v and w over the block's threads; the block totals land in *tv, *tw. One barrier: the scans of a wave run
+// in registers, and every thread adds the earlier waves' totals itself.
+__device__ __forceinline__ void block_exclusive_scan2(int& v, int& w, int2* s_tot, int* tv, int* tw) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int iv = v, iw = w;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int a = __shfl_up(iv, o), b = __shfl_up(iw, o);
+        iv += lane >= o ? a : 0;
+        iw += lane >= o ? b : 0;
     }
-    const int incl = s_scan[tid];
-    *total = s_scan[DISP_THREADS - 1];
+    if (lane == 63) s_tot[wave] = make_int2(iv, iw);
     __syncthreads();
-    return incl - v;
+    int sv = 0, sw = 0, pv = 0, pw = 0;
+#pragma unroll
+    for (int i = 0; i < DISP_WAVES; ++i) {
+        const int2 t = s_tot[i];
+        pv += i < wave ? t.x : 0;
+        pw += i < wave ? t.y : 0;
+        sv += t.x;
+        sw += t.y;
+    }
+    *tv = sv;
+    *tw = sw;
+    v = pv + iv - v;
+    w = pw + iw - w;
 }
 
 // Workgroup b places the pairs of chunk b = [b * 1024, b * 1024 + 1024). It reads every expert id (a few tens of
 // KB, L2-resident) to histogram both all pairs and the pairs before its chunk, so each workgroup knows where its
 // pairs go without a second launch or scratch memory: pos = start[e] + (pairs of e before the chunk) + (rank of
 // the pair among the chunk's pairs of e), ranks from ballots within a wave and per-wave counts across waves.
-// Workgroup 0 also writes the group tables.
+// Workgroup 0 also writes the groups; the padding of the tables is shared out by chunk. Bound by chains, not bytes: the ids are
+// read four at a time, a pair counts in one of two histograms (before the chunk, or not), and the scans take one barrier.
 __global__ void __launch_bounds__(DISP_THREADS) moe_dispatch_kernel(const int* __restrict__ eid, const float* __restrict__ wt, int n, int topk,
                                                                     int E, int gmax, int* __restrict__ tok_sorted, float* __restrict__ wt_sorted,
                                                                     int* __restrict__ inv, int* __restrict__ grp_expert, int* __restrict__ grp_start,
                                                                     int* __restrict__ n_groups) {
-    __shared__ int s_count[DISP_MAX_E], s_before[DISP_MAX_E], s_start[DISP_MAX_E], s_gbase[DISP_MAX_E];
+    __shared__ int s_count[DISP_MAX_E], s_before[DISP_MAX_E], s_start[DISP_MAX_E];
     __shared__ unsigned short s_wcnt[DISP_WAVES][DISP_MAX_E];
-    __shared__ int s_scan[DISP_THREADS];
+    __shared__ int2 s_tot[DISP_WAVES];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int c0 = blockIdx.x * DISP_THREADS;
     for (int e = tid; e < E; e += DISP_THREADS) { s_count[e] = 0; s_before[e] = 0; }
     for (int i = tid; i < DISP_WAVES * E; i += DISP_THREADS) s_wcnt[i / E][i % E] = 0;
     __syncthreads();
-    for (int p = tid; p < n; p += DISP_THREADS) {
-        const int e = eid[p];
-        if (e >= 0 && e < E) {
-            atomicAdd(&s_count[e], 1);
-            if (p < c0) atomicAdd(&s_before[e], 1);
-        }
+    for (int p = tid; p < n; p += 4 * DISP_THREADS) {
+        int e[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) e[i] = p + i * DISP_THREADS < n ? eid[p + i * DISP_THREADS] : -1;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (e[i] >= 0 && e[i] < E) atomicAdd(p + i * DISP_THREADS < c0 ? &s_before[e[i]] : &s_count[e[i]], 1);
     }
     __syncthreads();
-    // exclusive scans of the counts and of the group counts over experts: thread t owns a contiguous run
-    const int per = (E + DISP_THREADS - 1) / DISP_THREADS;
-    const int e0 = tid * per, e1 = min(E, e0 + per);
-    int cs = 0, gsum = 0;
-    for (int e = e0; e < e1; ++e) { cs += s_count[e]; gsum += (s_count[e] + gmax - 1) / gmax; }
-    int total_pairs, total_groups;
-    int run = block_exclusive_scan(cs, s_scan, &total_pairs);
-    int grun = block_exclusive_scan(gsum, s_scan, &total_groups);
-    for (int e = e0; e < e1; ++e) {
-        s_start[e] = run;
-        s_gbase[e] = grun;
-        run += s_count[e];
-        grun += (s_count[e] + gmax - 1) / gmax;
-    }
+    // exclusive scans of the counts and of the group counts over experts (one expert per thread: E <= 512)
+    const int cnt_e = tid < E ? s_count[tid] + s_before[tid] : 0;
+    int start_e = cnt_e, gbase_e = (cnt_e + gmax - 1) / gmax, total_pairs, total_groups;
+    block_exclusive_scan2(start_e, gbase_e, s_tot, &total_pairs, &total_groups);
+    if (tid < E) s_start[tid] = start_e;
     __syncthreads();
     // stable scatter of this chunk
     const unsigned long long below = (lane == 63) ? ~0ull >> 1 : ((1ull << lane) - 1ull);
@@ -131,21 +135,26 @@ __global__ void __launch_bounds__(DISP_THREADS) moe_dispatch_kernel(const int* _
         inv[p] = pos;
     }
     if (valid && !real) inv[p] = -1;   // a dropped pair (id outside [0, E)) has no sorted slot
-    if (blockIdx.x != 0) return;
     // groups of <= gmax pairs per expert, then padding (p2p.cu:124-131). The padding starts at the number of
     // placed pairs (n when every id is valid, as in the reference), so the last group ends there; the sorted slots
     // past it (left by dropped pairs) hold token 0 with weight 0.
-    for (int ee = tid; ee < E; ee += DISP_THREADS) {
-        const int ng = (s_count[ee] + gmax - 1) / gmax;
-        for (int g = 0; g < ng; ++g) { grp_expert[s_gbase[ee] + g] = ee; grp_start[s_gbase[ee] + g] = s_start[ee] + g * gmax; }
+    if (valid && p >= total_groups) {
+        grp_expert[p] = -1;
+        grp_start[p] = total_pairs;
     }
-    const int G = total_groups;
-    for (int g = G + tid; g < n; g += DISP_THREADS) { grp_expert[g] = -1; grp_start[g] = total_pairs; }
-    for (int q = total_pairs + tid; q < n; q += DISP_THREADS) { tok_sorted[q] = 0; wt_sorted[q] = 0.f; }
+    if (valid && p >= total_pairs) {
+        tok_sorted[p] = 0;
+        wt_sorted[p] = 0.f;
+    }
+    if (blockIdx.x != 0) return;
+    for (int g = 0; g * gmax < cnt_e; ++g) {   // tid < E
+        grp_expert[gbase_e + g] = tid;
+        grp_start[gbase_e + g] = start_e + g * gmax;
+    }
     if (tid == 0) {
-        grp_start[G] = total_pairs;
+        grp_start[total_groups] = total_pairs;
         grp_start[n] = total_pairs;
-        if (n_groups) *n_groups = G;
+        if (n_groups) *n_groups = total_groups;
     }
 }
 
