@@ -38,6 +38,21 @@ __device__ __forceinline__ void unpack8(const v4i v, float* f) {
     }
 }
 
+// fake_quant_fp8 of a thread's 8 values of a 32-group held by four consecutive lanes, as bf16
+__device__ __forceinline__ v4i fq8_octet(const float (&n)[8]) {
+    float amax = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(n[j]));
+    amax = fmaxf(amax, __shfl_xor(amax, 1, 4));
+    amax = fmaxf(amax, __shfl_xor(amax, 2, 4));
+    const int e = fq8_exponent(amax);
+    uint32_t oq[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        oq[j] = f32_to_bf16_bits(fq8_value(fq8_code(n[2 * j], e), e)) | (f32_to_bf16_bits(fq8_value(fq8_code(n[2 * j + 1], e), e)) << 16);
+    return v4i{(int)oq[0], (int)oq[1], (int)oq[2], (int)oq[3]};
+}
+
 // The x and y vectors of a thread's two 8-element pieces of row t (pieces tid and tid + 512, clamped to the row;
 // y NULL: x again, ignored), all four loads issued together.
 struct RowRaw { v4i x[2], y[2]; };
@@ -141,18 +156,8 @@ __global__ void __launch_bounds__(RT_THREADS) router_norm_kernel(const RouterArg
         *(v4i*)&s_xn[t][v * 8] = ov;
         if (rb == 0) {
             // four consecutive threads hold one FP8 group (the range and the row are multiples of 32 elements)
-            float amax = 0.f;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(n[j]));
-            amax = fmaxf(amax, __shfl_xor(amax, 1, 4));
-            amax = fmaxf(amax, __shfl_xor(amax, 2, 4));
-            const int e = fq8_exponent(amax);
-            uint32_t oq[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                oq[j] = f32_to_bf16_bits(fq8_value(fq8_code(n[2 * j], e), e)) | (f32_to_bf16_bits(fq8_value(fq8_code(n[2 * j + 1], e), e)) << 16);
             *(v4i*)(a.xn + (long long)t * a.ldn + k) = ov;
-            *(v4i*)(a.xq + (long long)t * a.ldq + k) = v4i{(int)oq[0], (int)oq[1], (int)oq[2], (int)oq[3]};
+            *(v4i*)(a.xq + (long long)t * a.ldq + k) = fq8_octet(n);
         }
     }
     __syncthreads();
@@ -197,9 +202,12 @@ extern "C" int dsv41_router_logits(const uint16_t* x, long long ldx, const uint1
 // g = l / 16. Each lane loads 16 bytes (4 consecutive k) of its row per 16-k block and uses them in 4 products
 // (product i takes k = 16 j + 4 g + i), with the matching activations from LDS, so every weight load is a full
 // 16-byte vector and each wave-load covers 16 rows x 64 contiguous bytes.
+// xq given: one more workgroup per k range writes xq = fake_quant_fp8(x) there (quant.py:34-54), which the experts take. It
+// runs beside the others and saves the quantiser's launch (4.5 us of a 48.5 us layer at one token).
 #define RF_THREADS 256
 __global__ void __launch_bounds__(RF_THREADS) router_f32w_kernel(const uint16_t* __restrict__ x, long long ldx, const float* __restrict__ G,
-                                                                 long long ldg, int E, int M, float* __restrict__ part) {
+                                                                 long long ldg, int E, int M, float* __restrict__ part,
+                                                                 uint16_t* __restrict__ xq, long long ldq) {
     __shared__ __align__(16) uint16_t s_x[RT_MAXM][RT_KC + 8];   // this workgroup's k range of the M rows, bf16
     __shared__ v4f s_acc[RF_THREADS / 64][64];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -207,6 +215,15 @@ __global__ void __launch_bounds__(RF_THREADS) router_f32w_kernel(const uint16_t*
     const int rb = blockIdx.x, ks = blockIdx.y;
     const int k0 = ks * RT_KC;
     const int col = lane & 15, kg = lane >> 4;
+    if (rb * 16 >= E) {   // the quantiser's workgroup: 8 values per thread, four consecutive threads one FP8 group
+        for (int i = tid; i < M * (RT_KC / 8); i += RF_THREADS) {
+            const int t = i / (RT_KC / 8), k = k0 + (i - t * (RT_KC / 8)) * 8;
+            float n[8];
+            unpack8(*(const v4i*)(x + (long long)t * ldx + k), n);
+            *(v4i*)(xq + (long long)t * ldq + k) = fq8_octet(n);
+        }
+        return;
+    }
     // stage the activations first (16 bytes per thread per step; rows past M are not read): they are L2 hits, and
     // behind the weight loads they would return only after them (loads return in issue order)
     for (int i = tid; i < M * (RT_KC / 8); i += RF_THREADS) {
@@ -248,11 +265,22 @@ __global__ void __launch_bounds__(RF_THREADS) router_f32w_kernel(const uint16_t*
     }
 }
 
-extern "C" int dsv41_router_logits_f32w(const uint16_t* x, long long ldx, const float* G, long long ldg, int E, int H, int M, float* part,
-                                        void* stream) {
+static int router_f32w(const uint16_t* x, long long ldx, const float* G, long long ldg, int E, int H, int M, float* part, uint16_t* xq,
+                       long long ldq, void* stream) {
     if (!x || !G || !part || M < 1 || M > RT_MAXM || E <= 0 || H <= 0 || (H % RT_KC) || ldx < H || ldg < H || (ldx & 7) ||
         (ldg & 3) || (((uintptr_t)x) & 15) || (((uintptr_t)G) & 15))
         return DSV41_EINVAL;
-    router_f32w_kernel<<<dim3((E + 15) / 16, H / RT_KC), RF_THREADS, 0, (hipStream_t)stream>>>(x, ldx, G, ldg, E, M, part);
+    router_f32w_kernel<<<dim3((E + 15) / 16 + (xq ? 1 : 0), H / RT_KC), RF_THREADS, 0, (hipStream_t)stream>>>(x, ldx, G, ldg, E, M, part, xq, ldq);
     return (int)hipGetLastError();
+}
+
+extern "C" int dsv41_router_logits_f32w(const uint16_t* x, long long ldx, const float* G, long long ldg, int E, int H, int M, float* part,
+                                        void* stream) {
+    return router_f32w(x, ldx, G, ldg, E, H, M, part, nullptr, 0, stream);
+}
+
+extern "C" int dsv41_router_logits_f32w_quant(const uint16_t* x, long long ldx, const float* G, long long ldg, int E, int H, int M, float* part,
+                                              uint16_t* xq, long long ldq, void* stream) {
+    if (!xq || xq == x || ldq < H || (ldq & 7) || (((uintptr_t)xq) & 15)) return DSV41_EINVAL;
+    return router_f32w(x, ldx, G, ldg, E, H, M, part, xq, ldq, stream);
 }

@@ -372,14 +372,14 @@ def prefill_up(xq: torch.Tensor, eid: torch.Tensor, wt: torch.Tensor, ex: Expert
     1149-1151 -> 1082-1087 us on one box. (The w2 launch keeps table order: its items are four times shorter, and
     largest first made it slower, 720 -> 746 us, in the same A/B.)"""
     from .hipkern import LIGHT_GROUP, moe_dispatch, tile_group
-    from .quant import quant_fp8_e8m0
+    from .quant import attached_codes, quant_fp8_e8m0
     dev = _lib.require_cuda(xq, eid, wt)
     T, H = xq.shape
     k = eid.shape[-1]
     P = T * k
     I = ex.I
     assert H == ex.H and xq.dtype == torch.bfloat16 and ex.E <= 512
-    xc, xs = quant_fp8_e8m0(xq)
+    xc, xs = attached_codes(xq, False) or quant_fp8_e8m0(xq)   # the operand xq was written with, or its codes (exact)
     light = tile_group(P, ex.E) == LIGHT_GROUP
     gmax = LIGHT_GROUP if light else PREFILL_GROUP
     tok_sorted, wt_sorted, inv, grp_expert, grp_start = moe_dispatch(eid, wt, k, ex.E, gmax, dev)
@@ -549,16 +549,21 @@ class MoEDecodeLayer:
 
 
 # --------------------------------------------------------------------------- the whole MoE layer (eager / prefill)
-def router_logits_f32w(x: torch.Tensor, G: torch.Tensor, part: torch.Tensor | None = None) -> torch.Tensor:
+def router_logits_f32w(x: torch.Tensor, G: torch.Tensor, part: torch.Tensor | None = None, xq: torch.Tensor | None = None) -> torch.Tensor:
     """Router logits with fp32 router weights G [E, H] for M <= 16 bf16 rows x (F.linear(x.float(), gate_w),
     model.py:392): fp32 [H / 1024, M, E] partial sums over k ranges of 1024, which gate_topk / moe_route_experts add
-    in part order."""
-    dev = _lib.require_cuda(x, G, part)
+    in part order. xq (bf16 [M, H]) receives fake_quant_fp8(x) in the same launch."""
+    dev = _lib.require_cuda(x, G, part, xq)
     M, H = x.shape
     E = G.shape[0]
     assert x.dtype == torch.bfloat16 and G.dtype == torch.float32 and G.shape[1] == H and G.stride(1) == 1 and x.stride(1) == 1
     part = torch.empty(H // 1024, M, E, dtype=torch.float32, device=dev) if part is None else part
     assert part.shape == (H // 1024, M, E) and part.is_contiguous()
+    if xq is not None:
+        assert xq.shape == (M, H) and xq.dtype == torch.bfloat16 and xq.stride(1) == 1
+        _lib.call("dsv41_router_logits_f32w_quant", _lib.ptr(x), x.stride(0), _lib.ptr(G), G.stride(0), E, H, M, _lib.ptr(part), _lib.ptr(xq),
+                  xq.stride(0), _lib.stream(dev))
+        return part
     _lib.call("dsv41_router_logits_f32w", _lib.ptr(x), x.stride(0), _lib.ptr(G), G.stride(0), E, H, M, _lib.ptr(part), _lib.stream(dev))
     return part
 
@@ -569,7 +574,7 @@ class MoE:
     scaled), x fake-quantised to FP8 (model.py:565), the routed FP4 experts, the shared expert (bf16, or FP8 w8.W8 as
     the checkpoint stores it), and
     y = bf16(sum_j w_j y2_j + shared) (model.py:589-591).
-      * <= 16 tokens (decode): the router GEMV on fp32 weights as split-K partial sums, then the two fused decode
+      * <= 16 tokens (decode): the router GEMV on fp32 weights as split-K partial sums with the FP8 quantisation of x, then the two fused decode
         launches (routing inside the up launch for one token; a bf16 shared expert rides in both launches when it fits
         them, else runs as its own launches first; an FP8 one runs first as two FP8 GEMM launches and a SwiGLU);
       * > 16 tokens (prefill): router logits and the shared expert's two products as plain library GEMMs (F.linear on
@@ -653,16 +658,15 @@ class MoE:
         T, H = x2.shape
         if T <= 16:
             b = self._buf(dev, T)
-            _lib.call("dsv41_quant_fp8", _lib.ptr(x2), 0, T, H, x2.stride(0), 0, None, None, _lib.ptr(b["xq"]), _lib.stream(dev))
-            router_logits_f32w(x2, self.gate_w, part=b["part"])
+            router_logits_f32w(x2, self.gate_w, part=b["part"], xq=b["xq"])   # and xq = fake_quant_fp8(x) (model.py:565)
             ys = self._shared_rows(b["xq"]) if self.shared is None and self.sh_w13 is not None else None
             moe_route_experts(b["xq"], b["part"], self.gate_bias, self.gate_temp, self.topk, self.route_scale, self.score_func, self._norm(),
                               self.ex, self.swiglu_limit, ys=ys, out=b["out"], eid_out=b["eid"], wt_out=b["wt"], shared=self.shared)
             self.last_routing = (b["eid"], b["wt"])
             return b["out"].view(shape)
-        from .quant import fake_quant_fp8
+        from .quant import fake_quant_codes
         wt, eid = self.gate(x2)
-        xq = fake_quant_fp8(x2)
+        xq = fake_quant_codes(x2)
         ys = self._shared_rows(xq) if self.sh_w13 is not None else None
         out = torch.empty(T, H, dtype=torch.bfloat16, device=dev)
         prefill_experts(xq, eid, wt, self.ex, self.swiglu_limit, ys=ys, out=out)

@@ -292,6 +292,11 @@ int dsv41_router_logits(const uint16_t* x, long long ldx, const uint16_t* y, lon
 int dsv41_router_logits_f32w(const uint16_t* x, long long ldx, const float* G, long long ldg, int E, int H, int M, float* part,
                              void* stream);
 
+/* dsv41_router_logits_f32w that also writes xq = fake_quant_fp8(x) (bf16 [M][ldq], quant.py:34-54) in the same launch. xq must
+ * not alias x; 16-byte aligned, ldq % 8 == 0. */
+int dsv41_router_logits_f32w_quant(const uint16_t* x, long long ldx, const float* G, long long ldg, int E, int H, int M, float* part,
+                                   uint16_t* xq, long long ldq, void* stream);
+
 /* The decode block's hyper-connection steps either side of the experts (hc <= 4 residual streams):
  * pre (fused2.hc_pre_norm_quant2, fused2.py:189-236): per row b, a = bf16(sum_h pre[b][h] * x[b][h]) (x bf16 [B][ldx], the
  * hc streams D apart; pre fp32 [B][ldp]), y = bf16(a * (1 / sqrt(mean(a^2) + eps)) * w) (w bf16 [D]), yq =
