@@ -628,12 +628,11 @@ __device__ __forceinline__ void prefill_item256(const PrefillArgs& a, const int 
 
     // ---- DMA descriptors: weight slots 2 w, 2 w + 1; token blocks 2 w, 2 w + 1 (two loads of 8 rows each); weight scales
     // (tiled: wave 0, 16 B per lane; row-major: waves 0-3, 4 slots each); the pairs' E8M0 words (waves 4-7, 64 each)
-    const int nbw0 = block_of(2 * wave, cb0), nbw1 = block_of(2 * wave + 1, cb0);
     const int a_pc = ((lane & 3) ^ (lane >> 4)) * 16;   // this lane's piece of row lane / 4
     auto a_off = [&](int nb) {
         return TILED ? (uint32_t)(nb * nk * 1024 + (lane >> 2) * 64 + a_pc) : (uint32_t)((nb * 16 + (lane >> 2)) * Kh + a_pc);
     };
-    const uint32_t a_voff0 = a_off(nbw0), a_voff1 = a_off(nbw1);
+    const uint32_t a_voff0 = a_off(block_of(2 * wave, cb0)), a_dn = TILED ? (uint32_t)(nk * 1024) : (uint32_t)(16 * Kh);   // slot 2 w + 1: the next block
     const int a_ks = TILED ? 1024 : 64;
     const uint32_t a_cs = TILED ? (uint32_t)(PV_DNB * nk * 1024) : (uint32_t)(PV_DNB * 16 * Kh);
     const int asb = TILED ? block_of(lane >> 2, cb0) : block_of(4 * (wave & 3) + (lane >> 4), cb0), asr = lane & 15;
@@ -651,7 +650,7 @@ __device__ __forceinline__ void prefill_item256(const PrefillArgs& a, const int 
     const int per_step = 2 + (lda ? 1 : 0) + (ldb0 ? 2 : 0) + (ldb1 ? 2 : 0) + (ldbs ? 1 : 0);
 
     const int lofs = col * 64 + ((kb ^ (col >> 2)) * 16);                                                     // weight slot
-    const int bofs0 = col * 128 + ((kb ^ (col >> 1)) * 16), bofs1 = col * 128 + (((4 + kb) ^ (col >> 1)) * 16);   // token block, k half 0 / 1
+    const int bofs0 = col * 128 + ((kb ^ (col >> 1)) * 16);   // token block, k half 0; half 1: ^ 64
     bool tb_on[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) tb_on[u] = 16 * (2 * u + ph) < m;
@@ -659,7 +658,7 @@ __device__ __forceinline__ void prefill_item256(const PrefillArgs& a, const int 
     v4i OA[4], OB0[8], OB1[8];
     uint32_t OSA, OSB[2];
     // per-lane LDS offsets within a stage: weight slots relative to slot_of[0], token blocks of this half, scales
-    const uint32_t lofs_a = (uint32_t)(P2_A + slot_of[0] * 1024 + lofs), lofs_b = (uint32_t)(P2_B + ph * 2048 + bofs0), lofs_b1 = (uint32_t)(P2_B + ph * 2048 + bofs1);
+    const uint32_t lofs_a = (uint32_t)(P2_A + slot_of[0] * 1024 + lofs), lofs_b = (uint32_t)(P2_B + ph * 2048 + bofs0);
     const uint32_t lofs_as = (uint32_t)(P2_AS + slot_of[0] * 64 + col * 4 + kb), lofs_bs = (uint32_t)(P2_BS + 16 * ph * 4 + col * 4 + kb);
     // Every read of a step is issued before any of them is used: the token blocks unconditionally (a block without
     // pairs reads stale bytes of its slot, which no MFMA takes) and each E8M0 byte into a register of its own, packed
@@ -667,7 +666,8 @@ __device__ __forceinline__ void prefill_item256(const PrefillArgs& a, const int 
     // eight serial round trips per step, the longest part of the step.)
     auto read_ops = [&](int st) {
         const uint32_t so = (uint32_t)st * P2_STAGE;
-        const uint32_t oa = lofs_a + so, ob = lofs_b + so, ob1 = lofs_b1 + so, osa = lofs_as + so, osb = lofs_bs + so;
+        const uint32_t oa = lofs_a + so, ob = lofs_b + so, ob1 = ob ^ 64u,   // k half 1: bofs1 = bofs0 ^ 64
+                        osa = lofs_as + so, osb = lofs_bs + so;
         uint32_t ab[4], bb[8];
         if (any_on) {   // wave-uniform: a wave whose half of the group is empty reads and computes nothing
 #pragma unroll
@@ -774,7 +774,7 @@ __device__ __forceinline__ void prefill_item256(const PrefillArgs& a, const int 
         auto issue_st = [&](int st) {
             uint8_t* so = smem + st * P2_STAGE;
             __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void*)(so + P2_A + 2 * wave * 1024), 16, a_voff0, iao, 0, 0);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void*)(so + P2_A + (2 * wave + 1) * 1024), 16, a_voff1, iao, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void*)(so + P2_A + (2 * wave + 1) * 1024), 16, a_voff0, iao + a_dn, 0, 0);
             if (lda) {
                 if (TILED) __builtin_amdgcn_raw_ptr_buffer_load_lds(sr, (lds_void*)(so + P2_AS), 16, as_voff, iso, 0, 0);
                 else __builtin_amdgcn_raw_ptr_buffer_load_lds(sr, (lds_void*)(so + P2_AS + wave * 256), 4, as_voff, iso, 0, 0);
@@ -879,9 +879,15 @@ __device__ __forceinline__ void prefill_item256(const PrefillArgs& a, const int 
 #define PL_B 17408
 #define PL_BS (PL_B + 128 * PL_T)
 #define PL_STAGE (PL_BS + 4 * PL_T)
+// QS (activation scale rows of whole 16-byte pieces): the pairs' E8M0 bytes come as one 16-byte piece per pair for four
+// k-steps, into two buffers behind the stages, with the loads of the first of them. One word per pair and k-step is a load of up
+// to 64 scattered lines for 256 bytes: w13 at 2048 tokens 918 -> 881 us without it (333 tokens level; the larger tiles,
+// which are not bound by the weights' stream, gained nothing and keep the words).
+#define PL_Q (PL_NS * PL_STAGE)
+#define PL_LDS(QS) (PL_NS * PL_STAGE + ((QS) ? 2 * 16 * PL_T : 0))
 
 // Column block cb of expert e for the m <= PL_T pairs p0 .. p0 + m - 1. alone: the expert's only pass over these rows.
-template <int MODE, int TILED>
+template <int MODE, int TILED, int QS>
 __device__ __forceinline__ void prefill_pass_light(const PrefillArgs& a, const int e, const int p0, const int m, const int cb, const bool alone) {
     constexpr int TH = PL_T / 32;   // token blocks per wave
     extern __shared__ __align__(16) uint8_t smem[];   // PL_NS stages of PL_STAGE bytes
@@ -933,7 +939,7 @@ __device__ __forceinline__ void prefill_pass_light(const PrefillArgs& a, const i
                                                      ((lane & 7) ^ (4 * (wave & 1) + (lane >> 4))) * 16 : 0u;
     const uint32_t bs_voff = (uint32_t)s_row[lane & (PL_T - 1)] * (uint32_t)a.ldxs;
     const bool ldb = 16 * tb_w < m, lda = TILED ? wave == 0 : wave < 4, ldbs = wave == 4;
-    const int per_step = 2 + (lda ? 1 : 0) + (ldb ? 1 : 0) + (ldbs ? 1 : 0);
+    const int per_step = 2 + (lda ? 1 : 0) + (ldb ? 1 : 0) + (ldbs && !QS ? 1 : 0);
 
     const int lofs = col * 64 + ((kb ^ (col >> 2)) * 16);                                                     // weight slot
     const int bofs0 = col * 128 + ((kb ^ (col >> 1)) * 16), bofs1 = col * 128 + (((4 + kb) ^ (col >> 1)) * 16);   // token block, k half 0 / 1
@@ -945,7 +951,7 @@ __device__ __forceinline__ void prefill_pass_light(const PrefillArgs& a, const i
     for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int u = 0; u < TH; ++u) acc[j][u] = v4f{0.f, 0.f, 0.f, 0.f};
-    auto compute = [&](int st) {
+    auto compute = [&](int st, int k) {
         if (!tb_on[0]) return;   // wave-uniform: no pair in this half
         const uint8_t* s = smem + st * PL_STAGE;
         v4i A[4], B0[TH], B1[TH];
@@ -960,7 +966,8 @@ __device__ __forceinline__ void prefill_pass_light(const PrefillArgs& a, const i
             const uint8_t* bt = s + PL_B + (2 * u + ph) * 2048;
             B0[u] = *(const v4i*)(bt + bofs0);
             B1[u] = *(const v4i*)(bt + bofs1);
-            bb[u] = s[PL_BS + (16 * (2 * u + ph) + col) * 4 + kb];
+            bb[u] = QS ? smem[PL_Q + ((k >> 2) & 1) * (16 * PL_T) + (16 * (2 * u + ph) + col) * 16 + 4 * (k & 3) + kb]
+                       : s[PL_BS + (16 * (2 * u + ph) + col) * 4 + kb];
         }
         const uint32_t sa = ab[0] | (ab[1] << 8) | (ab[2] << 16) | (ab[3] << 24);
         uint32_t sb = 0;
@@ -979,8 +986,12 @@ __device__ __forceinline__ void prefill_pass_light(const PrefillArgs& a, const i
     auto kloop = [&](auto ps_c, auto nt_c) __attribute__((always_inline)) {
         constexpr int PS = decltype(ps_c)::value, PL_AUX = decltype(nt_c)::value ? 2 : 0;
         uint32_t iao = 0, iso = 0, ixo = 0;
+        int is = 0;   // the step to issue
         auto issue_st = [&](int st) {
             uint8_t* so = smem + st * PL_STAGE;
+            if (QS && ldbs && (is & 3) == 0)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(xsr, (lds_void*)(smem + PL_Q + ((is >> 2) & 1) * (16 * PL_T)), 16, bs_voff, ixo >> 5, 0, 0);
+            ++is;
             __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void*)(so + PL_A + 2 * wave * 1024), 16, a_voff0, iao, 0, PL_AUX);
             __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void*)(so + PL_A + (2 * wave + 1) * 1024), 16, a_voff1, iao, 0, PL_AUX);
             if (lda) {
@@ -988,30 +999,30 @@ __device__ __forceinline__ void prefill_pass_light(const PrefillArgs& a, const i
                 else __builtin_amdgcn_raw_ptr_buffer_load_lds(sr, (lds_void*)(so + PL_AS + wave * 256), 4, as_voff, iso, 0, 0);
             }
             if (ldb) __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void*)(so + PL_B + wave * 1024), 16, b_voff, ixo, 0, 0);
-            if (ldbs) __builtin_amdgcn_raw_ptr_buffer_load_lds(xsr, (lds_void*)(so + PL_BS), 4, bs_voff, ixo >> 5, 0, 0);
+            if (!QS && ldbs) __builtin_amdgcn_raw_ptr_buffer_load_lds(xsr, (lds_void*)(so + PL_BS), 4, bs_voff, ixo >> 5, 0, 0);
             iao += a_ks;
             iso += as_ks;
             ixo += 128;
         };
         // step k in stage st; W: later steps of this wave in flight once its DMA of step k has landed
-        auto step = [&](int st, auto iss_c, auto w_c) __attribute__((always_inline)) {
+        auto step = [&](int k, int st, auto iss_c, auto w_c) __attribute__((always_inline)) {
             wait_vm_c<PS * decltype(w_c)::value>();
             __builtin_amdgcn_s_waitcnt((15) | (7 << 4) | (0 << 8) | (3 << 14));   // lgkmcnt(0): own LDS reads of step k - 1 done
             __builtin_amdgcn_s_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
             if constexpr (decltype(iss_c)::value != 0) issue_st(st == 0 ? PL_NS - 1 : st - 1);
-            compute(st);
+            compute(st, k);
         };
         issue_st(0);
         issue_st(1);
         int st = 0;
         for (int kk = 0; kk < nk - 2; ++kk) {
-            step(st, IntC<1>{}, IntC<1>{});
+            step(kk, st, IntC<1>{}, IntC<1>{});
             st = st == PL_NS - 1 ? 0 : st + 1;
         }
-        step(st, IntC<0>{}, IntC<1>{});
+        step(nk - 2, st, IntC<0>{}, IntC<1>{});
         st = st == PL_NS - 1 ? 0 : st + 1;
-        step(st, IntC<0>{}, IntC<0>{});
+        step(nk - 1, st, IntC<0>{}, IntC<0>{});
     };
     if (alone) {
         switch (per_step) {
@@ -1046,7 +1057,7 @@ __device__ __forceinline__ void prefill_pass_light(const PrefillArgs& a, const i
 }
 
 // Item L of the launch order (group, column block). A group of more than PL_T pairs takes several passes.
-template <int MODE, int TILED>
+template <int MODE, int TILED, int QS>
 __device__ __forceinline__ void prefill_item_light(const PrefillArgs& a, const int L) {
     const int jx = L >> 3, gi = jx / a.n_cb;
     const int g = item_group(a, gi * 8 + (L & 7)), cb = jx - gi * a.n_cb;
@@ -1058,14 +1069,14 @@ __device__ __forceinline__ void prefill_item_light(const PrefillArgs& a, const i
     const bool alone = p1 - p0 <= PL_T && (g == 0 || a.grp_expert[g - 1] != e) && (g + 1 >= a.G || a.grp_expert[g + 1] != e);
     for (int q = p0; q < p1; q += PL_T) {
         if (q > p0) __syncthreads();   // every wave has read the last pass's rows and operands
-        prefill_pass_light<MODE, TILED>(a, e, q, min(p1 - q, PL_T), cb, alone);
+        prefill_pass_light<MODE, TILED, QS>(a, e, q, min(p1 - q, PL_T), cb, alone);
     }
 }
 
-template <int MODE, int TILED>
+template <int MODE, int TILED, int QS>
 __global__ void __launch_bounds__(PG_THREADS, 4) prefill_gemm_light_kernel(const PrefillArgs a) {
     if (MODE == 2 && a.run_if && __builtin_amdgcn_readfirstlane(*a.run_if) == 0) return;
-    prefill_item_light<MODE, TILED>(a, (int)blockIdx.x);
+    prefill_item_light<MODE, TILED, QS>(a, (int)blockIdx.x);
 }
 
 // The prefill path's launch: each item takes the 256-pair tile when its group holds more than 128 pairs.
@@ -1095,18 +1106,26 @@ static int launch_prefill(PrefillArgs& a, int mode, int tiled, PrefillTile tile,
     const long long items = (long long)a.n_it * a.g_pad;   // a multiple of 8
     if (items > 0x7FFFFFFFll) return DSV41_EINVAL;
     const dim3 grid((unsigned)items), block(PG_THREADS);
-    const size_t lds = light ? (size_t)PL_NS * PL_STAGE : mixed ? (size_t)max(PV_NS * PV_STAGE, P2_NS * P2_STAGE) : (size_t)PV_NS * PV_STAGE;
-#define PV_LAUNCH(K, M, T)                                                                                            \
+    // light tile: four k-steps' E8M0 bytes of a pair as one 16-byte piece where the rows allow it
+    const bool qs = !(a.ldxs & 15) && !(((uintptr_t)a.xs) & 15) && a.K % 512 == 0;
+    const size_t lds = light ? (size_t)PL_LDS(qs) : mixed ? (size_t)max(PV_NS * PV_STAGE, P2_NS * P2_STAGE) : (size_t)PV_NS * PV_STAGE;
+#define PV_LAUNCH(K, ...)                                                                                            \
     do {                                                                                                          \
-        const hipError_t err = hipFuncSetAttribute((const void*)K<M, T>, hipFuncAttributeMaxDynamicSharedMemorySize, \
+        const hipError_t err = hipFuncSetAttribute((const void*)K<__VA_ARGS__>, hipFuncAttributeMaxDynamicSharedMemorySize, \
                                                    (int)lds);                                                     \
         if (err != hipSuccess) return (int)err;                                                                   \
-        K<M, T><<<grid, block, lds, st>>>(a);                                                                     \
+        K<__VA_ARGS__><<<grid, block, lds, st>>>(a);                                                                     \
     } while (0)
     if (light) {
-        if (mode == 0) { if (tiled) PV_LAUNCH(prefill_gemm_light_kernel, 0, 1); else PV_LAUNCH(prefill_gemm_light_kernel, 0, 0); }
-        else if (mode == 1) { if (tiled) PV_LAUNCH(prefill_gemm_light_kernel, 1, 1); else PV_LAUNCH(prefill_gemm_light_kernel, 1, 0); }
-        else { if (tiled) PV_LAUNCH(prefill_gemm_light_kernel, 2, 1); else PV_LAUNCH(prefill_gemm_light_kernel, 2, 0); }
+#define PL_LAUNCH(M)                                                                                              \
+    do {                                                                                                          \
+        if (tiled) { if (qs) PV_LAUNCH(prefill_gemm_light_kernel, M, 1, 1); else PV_LAUNCH(prefill_gemm_light_kernel, M, 1, 0); } \
+        else { if (qs) PV_LAUNCH(prefill_gemm_light_kernel, M, 0, 1); else PV_LAUNCH(prefill_gemm_light_kernel, M, 0, 0); }       \
+    } while (0)
+        if (mode == 0) PL_LAUNCH(0);
+        else if (mode == 1) PL_LAUNCH(1);
+        else PL_LAUNCH(2);
+#undef PL_LAUNCH
     } else if (mixed) {
         if (mode == 0) { if (tiled) PV_LAUNCH(prefill_gemm_mixed_kernel, 0, 1); else PV_LAUNCH(prefill_gemm_mixed_kernel, 0, 0); }
         else if (mode == 1) { if (tiled) PV_LAUNCH(prefill_gemm_mixed_kernel, 1, 1); else PV_LAUNCH(prefill_gemm_mixed_kernel, 1, 0); }
