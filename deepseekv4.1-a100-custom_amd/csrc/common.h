@@ -125,6 +125,20 @@ __device__ __forceinline__ float fq8_value_hw(uint32_t word, int e) {
     return __builtin_amdgcn_cvt_f32_fp8((int)word, B) * __uint_as_float((uint32_t)(127 + e) << 23);
 }
 
+// The fp32 values of a word of four codes, and two values of one group as a pair of bf16. A code's value (4 significant
+// bits, 2^-31 and up) is a bf16 value, so it is the upper half of its fp32 form; only a group of infinite amax (e = 128: its
+// values are infinities and NaN) takes the rounding's NaN rule.
+__device__ __forceinline__ void fq8_values4_hw(uint32_t word, int e, float* v) {
+    v[0] = fq8_value_hw<0>(word, e);
+    v[1] = fq8_value_hw<1>(word, e);
+    v[2] = fq8_value_hw<2>(word, e);
+    v[3] = fq8_value_hw<3>(word, e);
+}
+__device__ __forceinline__ uint32_t fq8_bf16_pair(float a, float b, int e) {
+    if (e > 127) return f32_to_bf16_bits(a) | (f32_to_bf16_bits(b) << 16);
+    return (__float_as_uint(a) >> 16) | (__float_as_uint(b) & 0xFFFF0000u);
+}
+
 // ------------------------------------------------------------------------------------------ two-term FP8 split
 // bf16 activations off the FP8 grid as two E4M3 x E8M0 terms per 32-group: hi = the per-32 rounding above, lo = the
 // residual x - hi (exact in fp32: x has 8 significant bits, hi 4, within 24 bits of each other) rounded the same way

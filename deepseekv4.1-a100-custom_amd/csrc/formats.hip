@@ -97,32 +97,35 @@ __global__ void __launch_bounds__(256) quant_fp8_vec_kernel(const void* __restri
     for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(f[i]));
     amax = fmaxf(amax, __shfl_xor(amax, 1, 2));
     const int e = fq8_exponent(amax);
-    uint32_t q[16];
+    uint32_t q[4];   // the codes in input order
 #pragma unroll
-    for (int i = 0; i < 16; ++i) q[i] = fq8_code(f[i], e);
+    for (int w = 0; w < 4; ++w) q[w] = fq8_code4_hw(f[4 * w], f[4 * w + 1], f[4 * w + 2], f[4 * w + 3], e);
     if (codes) {
         // natural position j holds input position (j & ~7) | bitrev3(j & 7) when the input is 8-k permuted
         uint32_t cw[4];
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
-            cw[w] = 0;
+            cw[w] = permuted ? 0 : q[w];
+            if (!permuted) continue;
 #pragma unroll
             for (int b = 0; b < 4; ++b) {
                 const int j = 4 * w + b;
-                const int src = permuted ? ((j & ~7) | ((j & 1) << 2) | (j & 2) | ((j >> 2) & 1)) : j;
-                cw[w] |= q[src] << (8 * b);
+                const int src = (j & ~7) | ((j & 1) << 2) | (j & 2) | ((j >> 2) & 1);
+                cw[w] |= ((q[src >> 2] >> (8 * (src & 3))) & 0xFFu) << (8 * b);
             }
         }
         *(v4i*)(codes + (long long)r * K + k0) = v4i{(int)cw[0], (int)cw[1], (int)cw[2], (int)cw[3]};
     }
     if (scales && (c & 1) == 0) scales[(long long)r * (K >> 5) + (c >> 1)] = (uint8_t)(e + 127);
     if (fq) {
+        float v[16];
+#pragma unroll
+        for (int w = 0; w < 4; ++w) fq8_values4_hw(q[w], e, v + 4 * w);
         if (x_f32) {
             v4i* dst = (v4i*)((float*)fq + (long long)r * K + k0);
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                dst[j] = v4i{__float_as_int(fq8_value(q[4 * j], e)), __float_as_int(fq8_value(q[4 * j + 1], e)),
-                             __float_as_int(fq8_value(q[4 * j + 2], e)), __float_as_int(fq8_value(q[4 * j + 3], e))};
+                dst[j] = v4i{__float_as_int(v[4 * j]), __float_as_int(v[4 * j + 1]), __float_as_int(v[4 * j + 2]), __float_as_int(v[4 * j + 3])};
         } else {
             v4i* dst = (v4i*)((uint16_t*)fq + (long long)r * K + k0);
 #pragma unroll
@@ -130,7 +133,7 @@ __global__ void __launch_bounds__(256) quant_fp8_vec_kernel(const void* __restri
                 uint32_t wd[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
-                    wd[i] = f32_to_bf16_bits(fq8_value(q[8 * j + 2 * i], e)) | (f32_to_bf16_bits(fq8_value(q[8 * j + 2 * i + 1], e)) << 16);
+                    wd[i] = fq8_bf16_pair(v[8 * j + 2 * i], v[8 * j + 2 * i + 1], e);
                 dst[j] = v4i{(int)wd[0], (int)wd[1], (int)wd[2], (int)wd[3]};
             }
         }
@@ -322,19 +325,19 @@ __global__ void __launch_bounds__(256) swiglu_quant_vec_kernel(const void* __res
     }
     amax = fmaxf(amax, __shfl_xor(amax, 1, 2));
     const int e = fq8_exponent(amax);
-    uint32_t q[16];
+    uint32_t cw[4];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) q[i] = fq8_code(h[i], e);
+    for (int j = 0; j < 4; ++j) cw[j] = fq8_code4_hw(h[4 * j], h[4 * j + 1], h[4 * j + 2], h[4 * j + 3], e);
     if (codes) {
-        uint32_t cw[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) cw[j] = q[4 * j] | (q[4 * j + 1] << 8) | (q[4 * j + 2] << 16) | (q[4 * j + 3] << 24);
         *(v4i*)(codes + (long long)r * inter + c0) = v4i{(int)cw[0], (int)cw[1], (int)cw[2], (int)cw[3]};
     }
     if (scales && (ch & 1) == 0) scales[(long long)r * (inter >> 5) + (ch >> 1)] = (uint8_t)(e + 127);
     if (hb) {
         // permute: column j of the chunk is stored at (j & ~7) | bitrev3(j & 7), a map that is its own inverse, so
         // output position k holds column perm(k)
+        float v[16];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) fq8_values4_hw(cw[j], e, v + 4 * j);
         v4i* dst = (v4i*)(hb + (long long)r * inter + c0);
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
@@ -344,7 +347,7 @@ __global__ void __launch_bounds__(256) swiglu_quant_vec_kernel(const void* __res
                 const int k0 = 8 * j + 2 * i, k1 = k0 + 1;
                 const int s0 = permute ? ((k0 & ~7) | ((k0 & 1) << 2) | (k0 & 2) | ((k0 >> 2) & 1)) : k0;
                 const int s1 = permute ? ((k1 & ~7) | ((k1 & 1) << 2) | (k1 & 2) | ((k1 >> 2) & 1)) : k1;
-                wd[i] = f32_to_bf16_bits(fq8_value(q[s0], e)) | (f32_to_bf16_bits(fq8_value(q[s1], e)) << 16);
+                wd[i] = fq8_bf16_pair(v[s0], v[s1], e);
             }
             dst[j] = v4i{(int)wd[0], (int)wd[1], (int)wd[2], (int)wd[3]};
         }

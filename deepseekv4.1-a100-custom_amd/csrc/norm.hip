@@ -69,11 +69,11 @@ __global__ void __launch_bounds__(NORM_THREADS) residual_rmsnorm_quant_kernel(co
     amax = fmaxf(amax, __shfl_xor(amax, 1, 4));
     amax = fmaxf(amax, __shfl_xor(amax, 2, 4));
     const int e = fq8_exponent(amax);
-    uint32_t qw[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-        qw[j] = f32_to_bf16_bits(fq8_value(fq8_code(v[2 * j], e), e)) | (f32_to_bf16_bits(fq8_value(fq8_code(v[2 * j + 1], e), e)) << 16);
-    *(v4i*)(xq + (long long)t * ldq + tid * 8) = v4i{(int)qw[0], (int)qw[1], (int)qw[2], (int)qw[3]};
+    float q[8];
+    fq8_values4_hw(fq8_code4_hw(v[0], v[1], v[2], v[3], e), e, q);
+    fq8_values4_hw(fq8_code4_hw(v[4], v[5], v[6], v[7], e), e, q + 4);
+    *(v4i*)(xq + (long long)t * ldq + tid * 8) = v4i{(int)fq8_bf16_pair(q[0], q[1], e), (int)fq8_bf16_pair(q[2], q[3], e),
+                                                     (int)fq8_bf16_pair(q[4], q[5], e), (int)fq8_bf16_pair(q[6], q[7], e)};
 }
 
 extern "C" int dsv41_residual_rmsnorm_quant(const uint16_t* x, long long ldx, const uint16_t* y, long long ldy, const uint16_t* w, float eps,
@@ -161,17 +161,18 @@ __global__ void __launch_bounds__(NORM_THREADS) hc_pre_norm_quant_kernel(const u
     amax = fmaxf(amax, __shfl_xor(amax, 1, 4));
     amax = fmaxf(amax, __shfl_xor(amax, 2, 4));
     const int e = fq8_exponent(amax);
-    uint32_t q[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) q[j] = f32_to_bf16_bits(fq8_value(fq8_code(v[j], e), e));
+    // codes and values by the conversion instructions (bit arithmetic for both: 21.7 -> 19.5 us for 1500 rows of 5120)
+    float q[8];
+    fq8_values4_hw(fq8_code4_hw(v[0], v[1], v[2], v[3], e), e, q);
+    fq8_values4_hw(fq8_code4_hw(v[4], v[5], v[6], v[7], e), e, q + 4);
     if (yq) {
-        const uint32_t qw[4] = {q[0] | (q[1] << 16), q[2] | (q[3] << 16), q[4] | (q[5] << 16), q[6] | (q[7] << 16)};
+        const uint32_t qw[4] = {fq8_bf16_pair(q[0], q[1], e), fq8_bf16_pair(q[2], q[3], e), fq8_bf16_pair(q[4], q[5], e), fq8_bf16_pair(q[6], q[7], e)};
         *(v4i*)(yq + (long long)b * ldq + tid * 8) = v4i{(int)qw[0], (int)qw[1], (int)qw[2], (int)qw[3]};
     }
     if (yqp) {
         // the 8-k permuted order (0, 4, 2, 6, 1, 5, 3, 7 within each 8, cukern.permute_x / fused2._perm8): slot s holds
         // element perm[s]
-        const uint32_t pw[4] = {q[0] | (q[4] << 16), q[2] | (q[6] << 16), q[1] | (q[5] << 16), q[3] | (q[7] << 16)};
+        const uint32_t pw[4] = {fq8_bf16_pair(q[0], q[4], e), fq8_bf16_pair(q[2], q[6], e), fq8_bf16_pair(q[1], q[5], e), fq8_bf16_pair(q[3], q[7], e)};
         *(v4i*)(yqp + (long long)b * ldqp + tid * 8) = v4i{(int)pw[0], (int)pw[1], (int)pw[2], (int)pw[3]};
     }
 }

@@ -46,11 +46,11 @@ __device__ __forceinline__ v4i fq8_octet(const float (&n)[8]) {
     amax = fmaxf(amax, __shfl_xor(amax, 1, 4));
     amax = fmaxf(amax, __shfl_xor(amax, 2, 4));
     const int e = fq8_exponent(amax);
-    uint32_t oq[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-        oq[j] = f32_to_bf16_bits(fq8_value(fq8_code(n[2 * j], e), e)) | (f32_to_bf16_bits(fq8_value(fq8_code(n[2 * j + 1], e), e)) << 16);
-    return v4i{(int)oq[0], (int)oq[1], (int)oq[2], (int)oq[3]};
+    float v[8];
+    fq8_values4_hw(fq8_code4_hw(n[0], n[1], n[2], n[3], e), e, v);
+    fq8_values4_hw(fq8_code4_hw(n[4], n[5], n[6], n[7], e), e, v + 4);
+    return v4i{(int)fq8_bf16_pair(v[0], v[1], e), (int)fq8_bf16_pair(v[2], v[3], e), (int)fq8_bf16_pair(v[4], v[5], e),
+               (int)fq8_bf16_pair(v[6], v[7], e)};
 }
 
 // The x and y vectors of a thread's two 8-element pieces of row t (pieces tid and tid + 512, clamped to the row;
