@@ -61,8 +61,23 @@ def test_light_tile_equals_the_larger_tiles(H, I, tiled):
         one = torch.ones(1, dtype=torch.int32, device=dev)
         hipkern.grouped_gemm_scatter(hi, his, ex.w13[:, :n], ex.s13[:, :n], ge, gs, tok, rows, wt, one, False, out, P, tiled,
                                      lo=(lo, los, flag), gmax=64 if suffix else 256)
-        got[suffix] = (hc, hs, y2, yt, out)
-    names = ("h codes", "h scales", "y2", "grouped", "scatter")
+        # FP8-grid x (no second term): the light tile stores the weighted rows of a new output itself; rows out of range are
+        # skipped, a given output is added to, shared rows take the atomic form (integers here: any order gives the same sums)
+        flag0 = torch.zeros(1, dtype=torch.int32, device=dev)
+        rows2 = rows.clone()
+        rows2[5], rows2[70] = -1, P
+        outs = []
+        for accum, distinct, ro, w in ((False, one, rows2, wt), (True, one, rows, wt), (False, flag0, rows // 4, None)):
+            o = torch.ones(P, n, device=dev) if accum else torch.zeros(P, n, device=dev)
+            sc = his if w is not None else torch.full_like(his, 127)
+            ws = ex.s13[:, :n] if w is not None else torch.full_like(ex.s13, 128)[:, :n]
+            ints = hi if w is not None else torch.randint(0, 2, hi.shape, generator=torch.Generator(device=dev).manual_seed(9), device=dev,
+                                                          dtype=torch.uint8) * 0x38      # 0 or 1.0
+            hipkern.grouped_gemm_scatter(ints, sc, ex.w13[:, :n], ws, ge, gs, tok, ro, wt if w is not None else torch.ones_like(wt), distinct, accum, o,
+                                         P, tiled, lo=(torch.zeros_like(lo), los, flag0), gmax=64 if suffix else 256)
+            outs.append(o)
+        got[suffix] = (hc, hs, y2, yt, out, *outs)
+    names = ("h codes", "h scales", "y2", "grouped", "scatter", "stored", "added", "atomic")
     for name, a, b in zip(names, got[""], got["_g64"]):
         assert torch.equal(a, b), name
     assert all(bool(t.any()) for t in got["_g64"])
