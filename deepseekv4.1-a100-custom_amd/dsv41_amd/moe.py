@@ -371,15 +371,22 @@ def prefill_up(xq: torch.Tensor, eid: torch.Tensor, wt: torch.Tensor, ex: Expert
     of up to PREFILL_GROUP the w13 launch takes them largest first (dsv41_group_order), so no long item starts near the end of it: configs[3] w13
     1149-1151 -> 1082-1087 us on one box. (The w2 launch keeps table order: its items are four times shorter, and
     largest first made it slower, 720 -> 746 us, in the same A/B.)"""
+    from .quant import quant_fp8_e8m0
+    _lib.require_cuda(xq, eid, wt)
+    _, H = xq.shape
+    assert H == ex.H and xq.dtype == torch.bfloat16 and ex.E <= 512
+    return _prefill_up_codes(*quant_fp8_e8m0(xq), eid, wt, ex, limit)
+
+
+def _prefill_up_codes(xc: torch.Tensor, xs: torch.Tensor, eid: torch.Tensor, wt: torch.Tensor, ex: ExpertWeights, limit: float) -> PrefillState:
+    """prefill_up of the FP8 operand (E4M3 codes [T, H], E8M0 bytes [T, H / 32])."""
     from .hipkern import LIGHT_GROUP, moe_dispatch, tile_group
-    from .quant import attached_codes, quant_fp8_e8m0
-    dev = _lib.require_cuda(xq, eid, wt)
-    T, H = xq.shape
+    dev = _lib.require_cuda(xc, xs, eid, wt)
+    T, H = xc.shape
     k = eid.shape[-1]
     P = T * k
     I = ex.I
-    assert H == ex.H and xq.dtype == torch.bfloat16 and ex.E <= 512
-    xc, xs = attached_codes(xq, False) or quant_fp8_e8m0(xq)   # the operand xq was written with, or its codes (exact)
+    assert H == ex.H and ex.E <= 512
     light = tile_group(P, ex.E) == LIGHT_GROUP
     gmax = LIGHT_GROUP if light else PREFILL_GROUP
     tok_sorted, wt_sorted, inv, grp_expert, grp_start = moe_dispatch(eid, wt, k, ex.E, gmax, dev)
@@ -666,9 +673,9 @@ class MoE:
             return b["out"].view(shape)
         from .quant import fake_quant_codes
         wt, eid = self.gate(x2)
-        xq = fake_quant_codes(x2)
+        xq, xc, xs = fake_quant_codes(x2)   # the FP8 operand with it: the w13 GEMM takes the codes
         ys = self._shared_rows(xq) if self.sh_w13 is not None else None
         out = torch.empty(T, H, dtype=torch.bfloat16, device=dev)
-        prefill_experts(xq, eid, wt, self.ex, self.swiglu_limit, ys=ys, out=out)
+        prefill_down(_prefill_up_codes(xc, xs, eid, wt, self.ex, self.swiglu_limit), self.ex, ys=ys, out=out)
         self.last_routing = (eid, wt)
         return out.view(shape)

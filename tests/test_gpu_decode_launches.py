@@ -31,9 +31,9 @@ def test_router_f32w_with_quantised_rows(M, H, E):
     assert L.dsv41_router_logits_f32w_quant(*args(_lib.ptr(xq), H - 8)) == -1
 
 
-def test_prefill_takes_the_recorded_operand():
-    """prefill_up on fake_quant_codes' result equals prefill_up on a copy of it (no record), and an in-place change drops the
-    record."""
+def test_prefill_operand_quantised_once():
+    """fake_quant_codes' operand gives what prefill_up quantises from its values, and prefill_up reads the values it is given: a
+    record left on a tensor whose bytes changed without a new version (library entry points write their `out` so) plays no part."""
     from dsv41_amd import moe, quant
     g = torch.Generator(device=DEV).manual_seed(5)
     E, H, I, k, T = 8, 512, 384, 2, 40
@@ -43,12 +43,13 @@ def test_prefill_takes_the_recorded_operand():
     x = torch.randn(T, H, generator=g, device=DEV).to(torch.bfloat16)
     eid = torch.randint(0, E, (T, k), generator=g, device=DEV, dtype=torch.int32)
     wt = torch.rand(T, k, generator=g, device=DEV)
-    xq = quant.fake_quant_codes(x)
-    assert torch.equal(xq, quant.fake_quant_fp8(x)) and quant.attached_codes(xq, False) is not None
+    xq, xc, xs = quant.fake_quant_codes(x)
+    assert torch.equal(xq, quant.fake_quant_fp8(x))
     y = moe.prefill_experts(xq, eid, wt, ex, 10.0)
-    assert torch.equal(y, moe.prefill_experts(xq.clone(), eid, wt, ex, 10.0))
-    xq.mul_(0)
-    assert quant.attached_codes(xq, False) is None and not moe.prefill_experts(xq, eid, wt, ex, 10.0).any()
+    assert torch.equal(y, moe.prefill_down(moe._prefill_up_codes(xc, xs, eid, wt, ex, 10.0), ex))
+    quant.attach_codes(xq, xc, xs)
+    xq.data.zero_()
+    assert quant.attached_codes(xq, False) is not None and not moe.prefill_experts(xq, eid, wt, ex, 10.0).any()
 
 
 @pytest.mark.parametrize("n,E,gmax", [(5000, 512, 64), (4096, 3, 256), (4097, 512, 1), (1025, 1, 7), (20000, 384, 256)])
