@@ -620,30 +620,47 @@ __device__ __forceinline__ uint32_t e4m3_e8m0_f32_bits(uint32_t c, uint32_t b) {
     return sign | (q + ((rem > half || (rem == half && (q & 1u))) ? 1u : 0u));
 }
 
-// one thread per 16 weights of a row: 16 B in, 32 B out (natural row-major bf16)
-__global__ void dequant_fp8_kernel(const uint8_t* __restrict__ W, long long ldw, int tiled, const uint8_t* __restrict__ S,
-                                   long long lds, int N, int K, uint16_t* __restrict__ out, long long ldo) {
-    const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int kq = K >> 4;
-    if (q >= (long long)N * kq) return;
-    const int n = (int)(q / kq), k16 = (int)(q % kq);
+// One thread per 16 weights of a row: 16 B in, 32 B out (natural row-major bf16). A wave takes 16 rows x 64 k, a stored tile
+// when tiled: four consecutive lanes hold a row's 64 k, so the wave reads whole lines of the tile and writes whole lines of
+// 16 output rows. Bound by the 3 bytes a weight moved; so the codes are decoded by instruction where the product is a normal
+// number (then exact, and its upper half the bf16 value): scale bytes 10 (2^-9 x 2^-117 = 2^-126) to 246 (448 x 2^119 <
+// 2^128), no NaN code. The rest takes the bit arithmetic. 32768 x 1280: 48.3 -> 25.9 us (2.6 -> 4.9 TB/s, a copy's rate; before: 16-byte
+// reads 256 bytes apart and the bit arithmetic for every code).
+__device__ __forceinline__ uint32_t dequant_pair_bits(uint32_t c0, uint32_t c1, uint32_t b) {
+    return f32_to_bf16_bits(__uint_as_float(e4m3_e8m0_f32_bits(c0, b))) | (f32_to_bf16_bits(__uint_as_float(e4m3_e8m0_f32_bits(c1, b))) << 16);
+}
+
+__global__ void __launch_bounds__(256) dequant_fp8_kernel(const uint8_t* __restrict__ W, long long ldw, int tiled, const uint8_t* __restrict__ S,
+                                                          long long lds, int N, int K, uint16_t* __restrict__ out, long long ldo) {
+    const int lane = threadIdx.x & 63;
+    const uint32_t ncb = ((uint32_t)K + 255u) >> 8, rb = blockIdx.x / ncb;   // workgroup: 16 rows x 256 k
+    const int n = (int)rb * 16 + (lane >> 2);
+    const int c = (int)(blockIdx.x - rb * ncb) * 4 + (int)(threadIdx.x >> 6), k16 = c * 4 + (lane & 3);
+    if (n >= N || k16 >= (K >> 4)) return;
     const uint8_t* src;
-    if (tiled) {
-        const int c = k16 >> 2, jj = k16 & 3;
-        src = W + (((long long)(n >> 4) * (K >> 6) + c) * 64 + jj * 16 + (n & 15)) * 16;
-    } else {
-        src = W + (long long)n * ldw + (long long)k16 * 16;
-    }
+    if (tiled) src = W + (((long long)rb * (K >> 6) + c) * 64 + (lane & 3) * 16 + (lane >> 2)) * 16;
+    else src = W + (long long)n * ldw + (long long)k16 * 16;
     const v4i w = *(const v4i*)src;
     const uint32_t b = S[(long long)(n >> 5) * lds + (k16 >> 1)];
     uint32_t o[8];
     const uint32_t words[4] = {(uint32_t)w.x, (uint32_t)w.y, (uint32_t)w.z, (uint32_t)w.w};
+    uint32_t nan = 0;   // bit 7 of a byte: its code is a NaN (0x7F or 0xFF)
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const uint32_t c0 = (words[i >> 1] >> (16 * (i & 1))) & 0xFFu, c1 = (words[i >> 1] >> (16 * (i & 1) + 8)) & 0xFFu;
-        const uint32_t lo = f32_to_bf16_bits(__uint_as_float(e4m3_e8m0_f32_bits(c0, b)));
-        const uint32_t hi = f32_to_bf16_bits(__uint_as_float(e4m3_e8m0_f32_bits(c1, b)));
-        o[i] = lo | (hi << 16);
+    for (int i = 0; i < 4; ++i) nan |= (words[i] & 0x7F7F7F7Fu) + 0x01010101u;
+    if (b >= 10u && b <= 246u && !(nan & 0x80808080u)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float v[4];
+            fq8_values4_hw(words[i], (int)b - 127, v);
+            o[2 * i] = (__float_as_uint(v[0]) >> 16) | (__float_as_uint(v[1]) & 0xFFFF0000u);
+            o[2 * i + 1] = (__float_as_uint(v[2]) >> 16) | (__float_as_uint(v[3]) & 0xFFFF0000u);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const uint32_t p = words[i >> 1] >> (16 * (i & 1));
+            o[i] = dequant_pair_bits(p & 0xFFu, (p >> 8) & 0xFFu, b);
+        }
     }
     v4i* dst = (v4i*)(out + (long long)n * ldo + (long long)k16 * 16);
     dst[0] = v4i{(int)o[0], (int)o[1], (int)o[2], (int)o[3]};
@@ -851,7 +868,7 @@ extern "C" int dsv41_dequant_fp8(const uint8_t* W, long long ldw, int tiled, con
                                  uint16_t* out, long long ldo, void* stream) {
     if (!W || !S || !out || N <= 0 || K <= 0 || (K & 15) || ldo < K || lds < (K + 31) / 32) return DSV41_EINVAL;
     if (tiled ? ((N & 15) || (K & 63) || ldw != K) : ldw < K) return DSV41_EINVAL;
-    const long long n16 = (long long)N * (K / 16);
-    dequant_fp8_kernel<<<(unsigned)((n16 + 255) / 256), 256, 0, (hipStream_t)stream>>>(W, ldw, tiled, S, lds, N, K, out, ldo);
+    const long long wgs = (((long long)N + 15) / 16) * (((long long)K + 255) / 256);
+    dequant_fp8_kernel<<<(unsigned)wgs, 256, 0, (hipStream_t)stream>>>(W, ldw, tiled, S, lds, N, K, out, ldo);
     return (int)hipGetLastError();
 }

@@ -66,6 +66,22 @@ def test_dequant_fp8_every_code_and_scale(tiled):
         assert np.array_equal(got[~nan], ref[~nan]), f"scale bytes {b0}..{b0 + 7}"
 
 
+@pytest.mark.parametrize("N,K,tiled,pad", [(1, 16, False, 0), (17, 48, False, 0), (33, 272, False, 16), (70, 4112, False, 48), (16, 64, True, 0),
+                                           (48, 320, True, 0), (528, 1280, True, 0)])
+def test_dequant_fp8_shapes(N, K, tiled, pad):
+    """Random codes (NaN codes among them) and scale bytes 0 .. 255 over partial 16-row and 256-k blocks and padded rows."""
+    from dsv41_amd import quant, w8
+    g = torch.Generator().manual_seed(N + K)
+    w = torch.randint(0, 256, (N, K + pad), generator=g, dtype=torch.uint8)
+    s = torch.randint(0, 256, ((N + 31) // 32, (K + 31) // 32), generator=g, dtype=torch.uint8)
+    wd = w8.tile(w).to(DEV) if tiled else w.to(DEV)[:, :K]
+    got = u16(quant.dequant_fp8_block(wd, s.to(DEV), tiled=tiled))
+    full = s.numpy().repeat(32, 0)[:N]
+    ref = np.concatenate([O.dequant_fp8_block(np.ascontiguousarray(w.numpy()[n:n + 1, :K]), full[n:n + 1]) for n in range(N)])
+    nan = np.isnan(O.bf16_bits_to_f32(ref))
+    assert np.array_equal(np.isnan(O.bf16_bits_to_f32(got)), nan) and np.array_equal(got[~nan], ref[~nan])
+
+
 @pytest.mark.parametrize("tiled", [False, True])
 @pytest.mark.parametrize("rows,N", [(4, 256), (16, 256), (64, 256), (16, 4112)])
 def test_fp8_gemm_decode_one_hot_exact(tiled, rows, N):
