@@ -24,14 +24,14 @@ from .quant import attached_codes, quant_fp8_split
 FP4_TILED = os.environ.get("DSV41_FP4_TILED", "1") == "1"  # experts stored in the tile_fp4 layout (cukern.py:231)
 FP4_W_MAX = 64                                              # tokens per group of the dispatch (cukern.py:232)
 
-_PERM8 = [0, 4, 2, 6, 1, 5, 3, 7]
-
 
 def permute_x(x: torch.Tensor) -> torch.Tensor:
     """bf16 [M, K] -> the 8-k permuted layout fp4_gemm_tc accepts (within every 8 k: 0,4,2,6,1,5,3,7),
-    cukern.py:224-227. A layout view, kept for drop-in compatibility (the HIP kernels take natural order)."""
+    cukern.py:224-227, kept for drop-in compatibility (the HIP kernels take natural order). The order swaps the outer two
+    of three bits of k, so it is one strided copy: an index list would be uploaded on every call, and the host would wait
+    for it behind the work in flight."""
     M, K = x.shape
-    return x.view(M, K // 8, 8)[:, :, _PERM8].reshape(M, K).contiguous()
+    return x.view(M, K // 8, 2, 2, 2).permute(0, 1, 4, 3, 2).reshape(M, K).contiguous()
 
 
 def _quant_x(x: torch.Tensor, permuted: bool, flag: bool = True):
