@@ -345,19 +345,23 @@ def fp8_rows_plan(M: int, N: int, K: int):
     """(activation rows per tile, K ranges) with which dsv41_fp8_gemm_rows multiplies M > 64 rows, or None where dequantising
     the weights and the library GEMM are faster.
     Tiles of 64 rows while they fit the CUs once, K split until about 256 workgroups (ranges of at least 1024 k); else tiles
-    of 128 up to 512 rows, and beyond them up to 1024 rows while one such tile per CU covers the product. us, dequantised +
-    library / tiles: 5120 x 8192 at 100 rows 72 / 33, 333 86 / 53, 700 106 / 77, 1400 143 / 132; 32768 x 1280 at 333 77 / 56,
-    700 104 / 102, 1400 147 / 186; 1280 x 5120 at 333 29 / 24, 700 35 / 34; 3328 x 7168 at 333 66 / 47, 700 80 / 68, 1400
-    99 / 105; 7168 x 1664 at 333 35 / 24, 700 40 / 40."""
+    of 128 up to 512 rows while at most three go to a CU, and beyond them up to 1024 rows while one per CU covers the product.
+    Beyond 512 rows with long weight rows they have to fill two thirds of the CUs: a tile's time is its chain over K, the
+    library's the product's size. us, dequantised + library / tiles (medians of graph replays over four weights): 5120 x 8192 at
+    128 rows 62 / 30, 333 69 / 57, 700 89 / 78, 900 101 / 116; 32768 x 1280 at 333 (three per CU) 55 / 52, 420 59 / 66;
+    16384 x 5120 at 512 117 / 91; 1280 x 5120 at 333 30 / 28, 512 34 / 32, 768 34 / 38; 3328 x 7168 at 333 52 / 50, 640 63 / 69,
+    900 72 / 71; 7168 x 1664 at 333 35 / 28, 640 36 / 40; 2048 x 2048 at 768 25 / 21."""
     if K % 64 or N % 8 or M > 1024:
         return None
     tn = (N + 127) // 128
     t64, t128 = tn * ((M + 63) // 64), tn * ((M + 127) // 128)
     if t64 <= 256:
-        tile, splits = 64, max(1, min(256 // t64, K // 1024, 8))
-    elif M <= 512 or t128 <= 256:
-        tile, splits = 128, 1
+        tile, splits, wgs = 64, max(1, min(256 // t64, K // 1024, 8)), t64
+    elif (M <= 512 and t128 <= 768) or t128 <= 256:
+        tile, splits, wgs = 128, 1, t128
     else:
+        return None
+    if M > 512 and K > 4096 and wgs < 176:
         return None
     # a range's scale bytes fit the kernel's 512
     return (tile, splits) if 2 * (-(-(K // 64) // splits)) <= 512 else None
