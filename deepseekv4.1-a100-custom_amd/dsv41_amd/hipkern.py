@@ -135,15 +135,22 @@ T128_MAX = 128   # pairs per group the 128-pair tile kernel computes
 LIGHT_GROUP = 64  # pairs per group of the light tile (two workgroups per CU, csrc/prefill.hip)
 TILE_GROUP = 256  # pairs per group of the larger tiles (128-pair tiles, 256-pair tiles for larger groups)
 LIGHT_PAIRS_PER_EXPERT = 48
+LIGHT_PAIRS = 2048
 
 
-def tile_group(n_pairs: int, n_experts: int) -> int:
+def tile_group(n_pairs: int, n_experts: int | None) -> int:
     """Pairs per group for the tile kernels: LIGHT_GROUP while the pairs average at most LIGHT_PAIRS_PER_EXPERT per expert,
     else TILE_GROUP. With few pairs per expert the launch is bound by the weight stream, which the light tile runs faster;
-    with more of them an expert's pairs fill several 64-pair groups that each stream its weights. w13 + w2 on either side,
-    larger tiles / light tile (7168 x 1664, 384 experts, top-8): 43 pairs per expert 1742 / 1623 us (uniform routing) and
-    1809 / 1818 (Zipf), 62 pairs per expert 2000 / 2170 and 2130 / 2185."""
-    return LIGHT_GROUP if n_pairs <= LIGHT_PAIRS_PER_EXPERT * n_experts else TILE_GROUP
+    with more of them an expert's pairs fill several 64-pair groups that each stream its weights. w13 + w2, larger tiles /
+    light tile in us, uniform and Zipf routing: 7168 x 1664, 384 experts, top-8 at 40 pairs per expert 1650 / 1525 and 1728 /
+    1665, 60 1926 / 1802 and 1957 / 1976, 90 2408 / 2623 and 2427 / 2463; 5120 x 2304, 384 experts, top-6 at 40 1632 / 1489 and
+    1678 / 1599, 60 1904 / 1745 and 1948 / 1940, 90 2293 / 2586; 4096 x 2048, 128 experts, top-8 at 48 440 / 364 and 470 / 423, 90
+    567 / 625.
+    n_experts None (not counted; the tables' bound of 512 says nothing): LIGHT_GROUP up to LIGHT_PAIRS pairs, where it is the
+    faster one for 2 to 384 experts and every form of output (7168 x 1664 over 2 experts 183 / 153, 4096 x 2048 over 128 325 /
+    270); 24,576 pairs added into a given output take 765 / 935 over 128 experts, 880 / 1047 over 2."""
+    few = n_pairs <= (LIGHT_PAIRS if n_experts is None else LIGHT_PAIRS_PER_EXPERT * n_experts)
+    return LIGHT_GROUP if few else TILE_GROUP
 
 
 def t128_ok(N: int, K: int, max_tokens: int) -> bool:

@@ -250,6 +250,25 @@ def test_grouped_fp4_gemm_scatter_forms(K):
     close(out2.cpu().numpy(), ref2, f"grouped_fp4_gemm shared rows (atomic) K={K}")
 
 
+@pytest.mark.parametrize("E,P,gmax", [(3, 2500, 256), (60, 2500, 64), (3, 700, 64)])
+def test_grouped_pairs_without_n_experts(E, P, gmax):
+    """GroupedPairs as the reference calls it, without n_experts: the launch takes its groups by the experts of the weights (or
+    of few pairs alone), not by the bound of the tables; the result is that of the counted dispatch bit for bit (distinct
+    output rows: stores, no atomics)."""
+    from dsv41_amd import moe_kernels, quant
+    N, K = 256, 512
+    w, s, _, _ = make_experts(E, K, N // 2, 47)
+    wtl, stl = quant.tile_fp4(w), quant.tile_fp4_scales(s)
+    x = quant.fake_quant_fp8(rand_x(100, K, 48).to(DEV))
+    rng = np.random.default_rng(49)
+    t = lambda a: torch.from_numpy(np.asarray(a, np.int32)).to(DEV)
+    args = (t(rng.integers(0, E, P)), t(rng.integers(0, 100, P)), t(np.arange(P)), torch.rand(P, device=DEV), 64)
+    free, counted = moe_kernels.GroupedPairs(*args), moe_kernels.GroupedPairs(*args, n_experts=E)
+    y = moe_kernels.grouped_fp4_gemm(x, wtl, stl, free, P, tiled=True)
+    assert free.tile_tables(E)[0] == gmax
+    assert torch.equal(y, moe_kernels.grouped_fp4_gemm(x, wtl, stl, counted, P, tiled=True)) and bool(y.any())
+
+
 def test_rows_distinct_flag():
     """dsv41_rows_distinct: 1 exactly when no two counted entries (the first n_placed, inside [0, out_rows)) repeat a
     row; 0 unchecked past its 2^20-row bitmap."""
