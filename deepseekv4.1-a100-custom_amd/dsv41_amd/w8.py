@@ -19,6 +19,7 @@ import os
 
 import torch
 import torch.nn.functional as F
+from torch.utils._device import DeviceContext
 
 from . import hipkern
 from .fused import fake_quant_fp8
@@ -115,14 +116,21 @@ class W8:
         return W8(torch.cat([w.w8 for w in ws], dim=0), torch.cat([w.s8 for w in ws], dim=0), permuted=True, tiled=ws[0].tiled)
 
 
+def _watched(x: torch.Tensor) -> bool:
+    """Whether something follows the torch operations on x, which a direct launch would pass by: gradients, forward mode, vmap,
+    tracing, autocast, tensor subclasses, dispatch and function modes (FLOP counters; a default device is none of them)."""
+    if type(x) is not torch.Tensor or torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._functorch.is_functorch_wrapped_tensor(x):
+        return True
+    if (torch.is_grad_enabled() and x.requires_grad) or torch.autograd.forward_ad._current_level >= 0 or torch.is_autocast_enabled():
+        return True
+    return torch._C._len_torch_dispatch_stack() > 0 or any(
+        type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(torch._C._len_torch_function_stack()))
+
+
 def _tiles_ok(x: torch.Tensor, w: "W8") -> bool:
     """Whether x . w^T can take the FP8 tiles: GPU tensors of 16-byte rows whose bytes 32-bit offsets reach, and nothing that
-    watches the call (gradients, forward-mode, vmap, tracing, autocast, tensor subclasses): those keep F.linear."""
-    if type(x) is not torch.Tensor or torch.compiler.is_compiling() or torch._C._functorch.is_functorch_wrapped_tensor(x):
-        return False
-    if (torch.is_grad_enabled() and x.requires_grad) or torch.autograd.forward_ad._current_level >= 0 or torch.is_autocast_enabled():
-        return False
-    return (x.device == w.w8.device and x.is_cuda and x.shape[1] == w.shape[1] and (x.data_ptr() % 16 == 0 or not x.is_contiguous())
+    watches the call; the others keep F.linear."""
+    return (not _watched(x) and x.device == w.w8.device and x.is_cuda and x.shape[1] == w.shape[1] and (x.data_ptr() % 16 == 0 or not x.is_contiguous())
             and w.w8.data_ptr() % 16 == 0 and x.numel() * 2 < 1 << 31 and 128 * w.shape[1] < 1 << 31)
 
 

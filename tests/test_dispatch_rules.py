@@ -9,3 +9,39 @@ def test_tile_group_counts_experts():
         assert tile_group(most * E, E) == LIGHT_GROUP and tile_group(most * E + 1, E) == TILE_GROUP
     assert tile_group(LIGHT_PAIRS, None) == LIGHT_GROUP
     assert tile_group(LIGHT_PAIRS + 1, None) == tile_group(most * 512, None) == TILE_GROUP
+
+
+def test_linear_w_sees_what_watches_a_call():
+    """w8._watched: what follows torch operations keeps w8.linear_w on F.linear; a default device does not."""
+    import torch
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from dsv41_amd.w8 import _watched
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    x = torch.ones(2, 4)
+    seen = []
+    note = lambda v: (seen.append(_watched(v)), v + 1)[1]
+    assert not _watched(x)
+    with torch.device("cpu"):
+        assert not _watched(x)
+        with Function():
+            assert _watched(x)
+    with Dispatch():
+        assert _watched(x)
+    torch.func.vmap(note)(x)
+    torch.func.jvp(note, (x,), (x,))
+    torch.jit.trace(note, x, check_trace=False)
+    torch.fx.experimental.proxy_tensor.make_fx(note)(x)
+    assert len(seen) == 4 and all(seen)
+    assert _watched(torch.nn.Parameter(x)) and _watched(x.clone().requires_grad_(True))
+    with torch.no_grad():
+        assert not _watched(x.clone().requires_grad_(True))

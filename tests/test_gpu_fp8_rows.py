@@ -105,6 +105,10 @@ def test_linear_w_rows_plan_and_watchers():
     assert xg.grad is not None
     out = torch.func.vmap(lambda r: w8.linear_w(r, W))(x.view(2, M // 2, K))
     assert torch.allclose(out.reshape(M, N).float(), lib.float(), rtol=2 ** -7, atol=1e-2 * lib.float().std().item())
+    from torch.utils.flop_counter import FlopCounterMode
+    with FlopCounterMode(display=False) as flops:
+        assert torch.equal(w8.linear_w(x, W), lib)
+    assert flops.get_total_flops() == 2 * M * N * K
     with torch.autocast("cuda", dtype=torch.float16):
         assert w8.linear_w(x, W).dtype == torch.float16
     g = torch.cuda.CUDAGraph()
