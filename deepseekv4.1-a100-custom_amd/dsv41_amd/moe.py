@@ -11,7 +11,9 @@ Decode (decode.py:316-372 experts_tc / moe2; model.py:554-591 MoE.__call__ for <
      out = bf16(y + ys) (fused2.py:490-495)
 Only the selected experts' weight bytes are read from HBM.
 
-Workspaces are allocated once per (device, shape) and reused, so a captured graph replays without allocating.
+Workspaces are allocated once per (device, shape) and reused, so a captured graph replays without allocating. Decode calls
+of one shape share them, whatever layer they are of, so such calls (and replays of graphs that hold them) are ordered one after
+another: on one stream, or with an event between two streams, and issued by one thread at a time.
 """
 from __future__ import annotations
 
@@ -588,7 +590,8 @@ class MoE:
         the GPU, as the reference runs them, model.py:392, 410-412; w8.py:102-103), gate_topk, then the prefill grouped
         GEMMs with the slot-ordered combine.
     Attribute names follow the reference (n_experts, topk, score_func, gate_temp, norm_topk_prob, route_scale,
-    swiglu_limit, gate_w, gate_bias, inter, sh_w13, sh_w2). Routing of the last call: last_routing."""
+    swiglu_limit, gate_w, gate_bias, inter, sh_w13, sh_w2). Routing of the last call: last_routing. The output and the routing
+    are the call's own tensors at every size; up to 16 tokens the work between shares its buffers (the module's docstring)."""
 
     def __init__(self, experts: ExpertWeights, gate_w: torch.Tensor, gate_bias: torch.Tensor | None = None, topk: int = 8,
                  score_func: str = "softmax", route_scale: float = 1.0, norm_topk_prob: bool = True, gate_temp: float = 1.0,
@@ -650,10 +653,8 @@ class MoE:
     def _buf(self, dev, T):
         b = self._bufs.get(T)
         if b is None:
-            H, E, k = self.dim, self.n_experts, self.topk
-            b = self._bufs[T] = {"xq": torch.empty(T, H, dtype=torch.bfloat16, device=dev), "out": torch.empty(T, H, dtype=torch.bfloat16, device=dev),
-                                 "part": torch.empty(H // 1024, T, E, dtype=torch.float32, device=dev),
-                                 "eid": torch.empty(T, k, dtype=torch.int32, device=dev), "wt": torch.empty(T, k, dtype=torch.float32, device=dev)}
+            b = self._bufs[T] = {"xq": torch.empty(T, self.dim, dtype=torch.bfloat16, device=dev),
+                                 "part": torch.empty(self.dim // 1024, T, self.n_experts, dtype=torch.float32, device=dev)}
         return b
 
     def __call__(self, x: torch.Tensor) -> torch.Tensor:
@@ -667,10 +668,13 @@ class MoE:
             b = self._buf(dev, T)
             router_logits_f32w(x2, self.gate_w, part=b["part"], xq=b["xq"])   # and xq = fake_quant_fp8(x) (model.py:565)
             ys = self._shared_rows(b["xq"]) if self.shared is None and self.sh_w13 is not None else None
+            out = torch.empty_like(x2)
+            eid = torch.empty(T, self.topk, dtype=torch.int32, device=dev)
+            wt = torch.empty(T, self.topk, dtype=torch.float32, device=dev)
             moe_route_experts(b["xq"], b["part"], self.gate_bias, self.gate_temp, self.topk, self.route_scale, self.score_func, self._norm(),
-                              self.ex, self.swiglu_limit, ys=ys, out=b["out"], eid_out=b["eid"], wt_out=b["wt"], shared=self.shared)
-            self.last_routing = (b["eid"], b["wt"])
-            return b["out"].view(shape)
+                              self.ex, self.swiglu_limit, ys=ys, out=out, eid_out=eid, wt_out=wt, shared=self.shared)
+            self.last_routing = (eid, wt)
+            return out.view(shape)
         from .quant import fake_quant_codes
         wt, eid = self.gate(x2)
         xq, xc, xs = fake_quant_codes(x2)   # the FP8 operand with it: the w13 GEMM takes the codes

@@ -1090,6 +1090,24 @@ def test_decode_fused_fp8_shared_expert(full_layer, M):
     close(bf16_vals(ys), bf16_vals(ys_w8), f"fused vs linear_w FP8 shared expert M={M}")
 
 
+@pytest.mark.parametrize("T", [1, 3, 16, 17])
+def test_moe_layer_results_are_the_calls_own(T):
+    """A result and its routing that the caller holds stay what they were when the layer is called again, on decode and
+    prefill sizes alike."""
+    from dsv41_amd import moe
+    E, H, I, k = 32, 1024, 384, 4
+    ex = to_ex(*make_experts(E, H, I, 1500 + T), True)
+    gate_w = torch.randn(E, H, generator=torch.Generator(device=DEV).manual_seed(T), device=DEV) / H ** 0.5
+    layer = moe.MoE(ex, gate_w, topk=k, swiglu_limit=10.0)
+    xa, xb = (rand_x(T, H, 1600 + i).to(DEV).view(1, T, H) for i in range(2))
+    ya = layer(xa)
+    held = (ya, *layer.last_routing)
+    copies = [t.clone() for t in held]
+    yb = layer(xb)
+    assert ya.shape == xa.shape and not torch.equal(yb, ya)
+    assert all(torch.equal(t, c) for t, c in zip(held, copies))
+
+
 @pytest.mark.parametrize("T", [1, 3, 40])
 def test_moe_layer_class(T):
     """model.MoE.__call__'s surface (moe.MoE): fp32 router weights, sigmoid gate with bias and route scale, FP8 x, routed
