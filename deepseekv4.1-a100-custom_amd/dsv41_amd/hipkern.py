@@ -350,25 +350,41 @@ def fp8_gemm_tc(x: torch.Tensor, w8: torch.Tensor, s8: torch.Tensor, group_cols:
 
 def fp8_rows_plan(M: int, N: int, K: int):
     """(activation rows per tile, K ranges) with which dsv41_fp8_gemm_rows multiplies M > 64 rows, or None where dequantising
-    the weights and the library GEMM are faster.
-    Tiles of 64 rows while they fit the CUs once, K split until about 256 workgroups (ranges of at least 1024 k); else tiles
-    of 128 up to 512 rows while at most three go to a CU, and beyond them up to 1024 rows while one per CU covers the product.
-    Beyond 512 rows with long weight rows they have to fill two thirds of the CUs: a tile's time is its chain over K, the
-    library's the product's size. us, dequantised + library / tiles (medians of graph replays over four weights): 5120 x 8192 at
-    128 rows 62 / 30, 333 69 / 57, 700 89 / 78, 900 101 / 116; 32768 x 1280 at 333 (three per CU) 55 / 52, 420 59 / 66;
-    16384 x 5120 at 512 117 / 91; 1280 x 5120 at 333 30 / 28, 512 34 / 32, 768 34 / 38; 3328 x 7168 at 333 52 / 50, 640 63 / 69,
-    900 72 / 71; 7168 x 1664 at 333 35 / 28, 640 36 / 40; 2048 x 2048 at 768 25 / 21."""
+    the weights and the library GEMM are faster. A tile's time is its chain over K, the library's the product's size.
+    us below: medians of graph replays over weights larger than the last-level cache.
+      * Small weights have too few tiles for their chains, unless K is short or falls into several ranges. dequantised + library /
+        tiles: 856 x 1280 at 65 rows 11.0 / 14.2, 856 x 2560 at 160 15.5 / 18.1, 2048 x 1280 at 160 13.3 / 14.8, 512 x 1984 at 333
+        17.4 / 18.8, 656 x 1216 at 640 14.7 / 15.3; on the other side of the lines 3000 x 1280 at 65 14.6 / 14.4, 2048 x 1280 at 333
+        16.3 / 15.1, 1280 x 1280 at 420 17.1 / 15.3, 4096 x 768 at 65 14.1 / 11.9, 512 x 5120 at 160 18.1 / 17.2.
+      * Tiles of 64 rows while they are at most 256, K in ranges of at least 1024 k. The weight tiles are dealt out to 8 XCDs of 32
+        CUs, and the ranges are as many as leave one tile to a CU on the XCD with the most of them: 1280 x 5120 (10 weight
+        tiles, two on two XCDs) at 256 rows in 5 / 4 ranges 25.6 / 20.3, 1280 x 2560 at 640 in 2 / 1 26.9 / 22.8, 2176 x 4096 at
+        160 in 4 / 3 23.9 / 20.5, 3328 x 7168 at 160 in 3 / 2 35.8 / 32.7. From K = 6144 on two ranges pay also where they put
+        two tiles on a CU: 5120 x 8192 at 256 in 1 / 2 56.9 / 52.1, 3000 x 7168 at 333 49.2 / 46.7 (6952 x 7232 at 160 52.5 / 55.8,
+        so up to 40 weight tiles).
+      * Tiles of 128 up to 512 rows while at most three go to a CU (dequantised + library / tiles: 32768 x 1280 at 333 55 / 52, 420 59 /
+        66; 16384 x 5120 at 512 117 / 91), and beyond them up to 1024 rows while one per CU covers the product. Beyond 512 rows with
+        long weight rows they have to fill two thirds of the CUs (5120 x 8192 at 700 89 / 78, 900 101 / 116; 1280 x 5120 at 768
+        34 / 38), and 64-row tiles may not share one (2176 x 7168 at 768 50.2 / 65.1).
+    The line is not the best one everywhere: 4608 x 5120 at 420 / 640 rows 52.3 / 53.2 and 55.0 / 58.6, 2992 x 5376 at 900 51.1 /
+    60.1, 8672 x 2112 at 512 40.4 / 47.4; three ranges of 128-row tiles, which it does not use, take 65 for 5120 x 8192 at 420
+    against 76 in one."""
     if K % 64 or N % 8 or M > 1024:
         return None
+    if 1088 < K <= 3072 and N * K < (2_700_000 if M <= 192 else 1_570_000 if M <= 384 else 1_050_000):
+        return None
     tn = (N + 127) // 128
-    t64, t128 = tn * ((M + 63) // 64), tn * ((M + 127) // 128)
-    if t64 <= 256:
-        tile, splits, wgs = 64, max(1, min(256 // t64, K // 1024, 8)), t64
-    elif (M <= 512 and t128 <= 768) or t128 <= 256:
-        tile, splits, wgs = 128, 1, t128
+    t64, t128 = (M + 63) // 64, (M + 127) // 128
+    if tn * t64 <= 256:
+        xcd = (tn + 7) // 8 * t64   # tiles of the XCD with the most of them
+        fit = 2 if 16 < xcd <= 32 and K >= 6144 and tn <= 40 else 32 // xcd
+        tile, splits = 64, max(1, min(fit, K // 1024, 8))
+        filled = tn * t64 >= 176 and xcd <= 32
+    elif (M <= 512 and tn * t128 <= 768) or tn * t128 <= 256:
+        tile, splits, filled = 128, 1, tn * t128 >= 176
     else:
         return None
-    if M > 512 and K > 4096 and wgs < 176:
+    if M > 512 and K > 4096 and not filled:
         return None
     # a range's scale bytes fit the kernel's 512
     return (tile, splits) if 2 * (-(-(K // 64) // splits)) <= 512 else None

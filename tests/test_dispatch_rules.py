@@ -45,3 +45,24 @@ def test_linear_w_sees_what_watches_a_call():
     assert _watched(torch.nn.Parameter(x)) and _watched(x.clone().requires_grad_(True))
     with torch.no_grad():
         assert not _watched(x.clone().requires_grad_(True))
+
+
+def test_fp8_rows_plan():
+    """The tiles of w8.linear_w past 64 rows: not for small weights with an unsplit chain over K, and as many K ranges as leave
+    one 64-row tile to a CU of the XCD (of 8, with 32 CUs) that has the most weight tiles; two where K is long."""
+    from dsv41_amd.hipkern import fp8_rows_plan
+    for M, N, K in ((65, 856, 1280), (160, 856, 2560), (333, 512, 1984), (640, 656, 1216), (160, 2048, 1280)):
+        assert fp8_rows_plan(M, N, K) is None
+    for (M, N, K), plan in {(640, 1280, 2560): (64, 1), (256, 1280, 5120): (64, 4), (160, 3328, 7168): (64, 2), (160, 2176, 4096): (64, 3),
+                            (256, 5120, 8192): (64, 2), (65, 4096, 768): (64, 1), (160, 512, 5120): (64, 5)}.items():
+        assert fp8_rows_plan(M, N, K) == plan
+    for M in (65, 100, 192, 193, 320, 500, 640, 1000):
+        for N in range(256, 9000, 424):
+            for K in range(512, 16384, 704):
+                plan = fp8_rows_plan(M, N, K)
+                if plan is None or plan[0] == 128:
+                    continue
+                tn, nk = (N + 127) // 128, K // 64
+                load = (tn + 7) // 8 * ((M + 63) // 64) * plan[1]
+                assert 1 <= plan[1] <= 8 and 2 * -(-nk // plan[1]) <= 512
+                assert plan[1] == 1 or load <= 32 or (plan[1] == 2 and K >= 6144 and load <= 64)
