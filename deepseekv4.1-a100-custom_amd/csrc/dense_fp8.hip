@@ -712,23 +712,39 @@ static bool fp8_lds_operands_ok(const Fp8Args& a, int tiled, int rows) {
 }
 
 // Row blocks per workgroup of the loader-wave kernel for this call (8: the 128-row tiles; 0: fp8_gemm_kernel). Both sides in us,
-// fp8_gemm_kernel first unless said otherwise; medians of 20 graph replays.
-//  * fewer than 256 row blocks (one per workgroup): long rows only. 3328 x 7168 at 16 / 8 rows 10.9 -> 8.9 / 10.1 -> 8.4,
-//    1280 x 5120 at 48 18.9 -> 9.8; 2048 x 512 at 32 4.1 / 4.2, so short rows (K < 1024; up to 16 tokens K < 2048) stay.
+// fp8_gemm_kernel first unless said otherwise; medians of graph replays over weights larger than the last-level cache.
+//  * fewer than 256 row blocks (one per workgroup): long rows only. 1280 x 5120 at 48 18.9 -> 9.8, 3328 x 7168 at 16 10.8 -> 9.2;
+//    2048 x 512 at 32 4.1 / 4.2, so short rows (K < 1024; up to 16 tokens K < 2048) stay. A few tokens load too little for the
+//    loader waves to pay: 3328 x 7168 at 5 7.9 / 8.4, 2992 x 5376 at 5 6.7 / 7.3, 1080 x 3008 at 7 5.65 / 5.94, 4000 x 3520 at 8 5.72 /
+//    5.96, against 1600 x 7168 at 8 8.16 / 7.87, 4000 x 5120 at 12 8.07 / 7.82. Token rows a multiple of 8 KB apart (K % 4096 == 0)
+//    collide in fp8_gemm_kernel's loads, so up to 192 blocks it loses from 5 on (1280 x 8192 at 5 / 8 7.99 -> 7.80 / 8.82 -> 7.85).
 //  * up to 512: two. 5120 x 8192 at 32 21.4 -> 15.1 (one: 21.2, four: 19.9). Up to 16 tokens the gain is small (5120 x 8192 14.6 ->
 //    13.1) and ends before 512 blocks (8192 x 2048 6.5 / 6.6).
 //  * more: four. 16384 x 5120 at 48 43.2 -> 22.1 (two: 27.6), 16384 x 2048 21.9 -> 13.5. Up to 16 tokens long rows only
-//    (16384 x 5120 22.8 -> 17.7, 16384 x 2048 10.3 / 10.3).
+//    (16384 x 5120 22.8 -> 17.7, 16384 x 2048 10.3 / 10.3). With K % 4096 == 0 the weight streams of many blocks collide, so few
+//    tokens take them up to 640 blocks (9600 x 4096 at 16 15.9 -> 14.4; 16384 x 4096 at 16 16.7 / 19.2, 16384 x 8192 29.8 / 36.9, 64000 x
+//    4096 54.2 / 62.1), and past 896 blocks some more tokens are needed (14000 x 8192 at 17 31.7 ->
+//    29.8, 16384 x 8192 33.0 / 38.0, at 24 36.9 / 37.4).
+//    Beyond 1024 blocks they are more workgroups than CUs, one to a CU, and the last of them leave most of the chip idle; so up to
+//    16 tokens only from 1536 blocks and 11 tokens on (24592 x 5120 at 9 / 16 27.9 / 31.0 and 34.1 / 32.4, 28800 x 5120 at 16 38.2 ->
+//    32.4). Below 1536 blocks not with few tokens and short rows either: 20800 x 768 at 32 12.8 / 13.6, 20800 x 1280 at 24 / 32 14.8 /
+//    15.3 and 16.5 / 16.3, 24000 x 2048 at 20 / 28 18.1 / 19.3 and 20.0 / 20.0, 24000 x 4096 at 18 28.0 / 30.3, 16640 x 2560 at 20
+//    21.3 -> 19.9; 24000 x 1472 at 40 25.3 -> 17.7.
 //  * 192 and more 128-row tiles with short rows: the tiles, whose activations are read once per 128 weight rows. 32768 x 1280 at
 //    48 / 64 33.3 -> 15.2 / 38.6 -> 17.2 (four blocks: 18.5 / 22.2), 24576 x 1280 at 48 25.4 -> 15.1 (17.4).
 static int fp8_stream_blocks(const Fp8Args& a, int nb) {
     if (a.M <= 4 || a.nk > 64 * FS_SW) return 0;
-    const bool few = a.M <= 16;
-    if (nb < 256) return a.nk >= (few ? 32 : 16) ? 1 : 0;
+    const bool few = a.M <= 16, collide = a.nk % 64 == 0;
+    if (nb < 256) {
+        const int least = nb <= 192 ? (collide ? 5 : 8) : a.nk >= 64 ? 8 : 12;
+        return few ? (a.nk >= 32 && a.M >= least ? 1 : 0) : a.nk >= 16 ? 1 : 0;
+    }
     if (few && a.M <= 8) return 0;
     if (nb <= 512) return !few || (nb <= 448 && a.nk >= 24) ? 2 : 0;
-    if (few) return a.nk >= 64 ? 4 : 0;
-    return nb >= 192 * 8 && a.nk <= 40 ? 8 : 4;
+    if (few) return a.nk >= 64 && (collide ? nb <= 640 : nb <= 1024 || (nb >= 1536 && a.M >= 11)) ? 4 : 0;
+    if (nb >= 192 * 8) return a.nk <= 40 ? 8 : 4;
+    const int most = nb <= 1024 ? (collide && nb > 896 ? 20 : 16) : a.nk >= 40 ? (collide ? 24 : 16) : a.nk >= 32 ? 24 : a.nk >= 16 ? 28 : 32;
+    return a.M > most ? 4 : 0;   // up to `most` tokens fp8_gemm_kernel
 }
 
 template <int NS, int MT, int RB, int TILED>

@@ -32,7 +32,8 @@ def _close(got, ref, what):
 UP_TO_64 = [(5, 1280, 2048, 0), (16, 1000, 4160, 0), (17, 2064, 1024, 0), (33, 4080, 1088, 0), (64, 3328, 7168, 0), (48, 512, 5120, 0),
             (9, 4112, 2304, 0), (16, 7168, 1664, 0), (31, 4104, 1280, 0), (49, 8192, 1024, 0), (64, 5128, 2112, 0),
             (16, 10240, 4096, 0), (33, 8208, 1024, 0), (64, 12296, 1088, 0), (17, 24576, 1024, 0), (40, 24600, 1088, 0), (64, 32768, 192, 0),
-            (20, 4096, 1024, 32), (20, 4096, 1024, 16), (50, 16384, 1024, 64), (20, 24576, 1024, 128)]
+            (20, 4096, 1024, 32), (20, 4096, 1024, 16), (50, 16384, 1024, 64), (20, 24576, 1024, 128),
+            (5, 1280, 4096, 0), (8, 3072, 2112, 0), (12, 3344, 2112, 0), (11, 24592, 4160, 0), (33, 16400, 768, 0)]
 
 
 @pytest.mark.parametrize("tiled", [True, False])
