@@ -1,6 +1,7 @@
 """The 64-pair tile of the prefill kernels (dsv41_prefill_up_g64 / _down_g64, dsv41_fp4_grouped_gemm_t64 / _scatter_g64) at
 the edges of its range: group sizes either side of a token block and of the tile (larger groups in passes), experts with one
-group and with several, both weight layouts, the shortest k-loops. Every pair's row is the same sum in the same order as on
+group and with several, both weight layouts, the shortest k-loops; and with the pairs' scale bytes in one load for four k-steps
+(K % 512 == 0) over one, two, three and four such loads, whose two buffers switch at the second and are filled again from the third on. Every pair's row is the same sum in the same order as on
 the larger tiles (which are checked against the oracle in test_gpu_moe.py), so the results are equal bit for bit."""
 import numpy as np
 import pytest
@@ -32,7 +33,7 @@ def _setup(H, I, tiled, seed):
 
 
 @pytest.mark.parametrize("tiled", [True, False])
-@pytest.mark.parametrize("H,I", [(512, 384), (768, 640)])
+@pytest.mark.parametrize("H,I", [(512, 384), (768, 640), (1024, 1536), (1536, 1024), (2048, 512)])
 def test_light_tile_equals_the_larger_tiles(H, I, tiled):
     from dsv41_amd import _lib, hipkern, quant
     print(f"light tile H={H} I={I} tiled={tiled}", flush=True)

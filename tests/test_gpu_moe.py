@@ -148,10 +148,10 @@ def test_grouped_fp4_gemm_atomic_rows(block_m):
 
 
 def test_big_groups_on_the_128_pair_tile_kernel():
-    """Groups of more than 16 pairs: cukern.fp4_gemm_tc (max_tokens 64, cukern.FP4_W_MAX) and moe_kernels.grouped_fp4_gemm
-    (block_m 64, the reference's prefill call, model.py:584-589) run on the 128-pair tile kernel; results equal the
-    textbook oracle, with repeated output rows (atomic sums), a group over the 64-pair cap split by the dispatch, and
-    dropped (out-of-range) expert ids."""
+    """Groups of more than 16 pairs on the tile kernels: cukern.fp4_gemm_tc with max_tokens 64 (cukern.FP4_W_MAX; the 64-pair tile)
+    and 128 (the 128-pair tile), and moe_kernels.grouped_fp4_gemm (block_m 64, the reference's prefill call, model.py:584-589; 50
+    pairs per expert: the larger tiles); results equal the textbook oracle, with repeated output rows (atomic sums), a popular
+    expert, and dropped (out-of-range) expert ids."""
     from dsv41_amd import hipkern, moe_kernels, quant
     E, N, K = 6, 512, 768
     w, s, _, _ = make_experts(E, K, N // 2, 21)
@@ -169,7 +169,14 @@ def test_big_groups_on_the_128_pair_tile_kernel():
     got = hipkern.fp4_gemm_tc(hipkern.permute_x(x), wtl, stl, ge, gs, tok, P, 64)
     ref = O.grouped_gemm(bf16_vals(x), w.cpu().numpy(), s.cpu().numpy(), ge.cpu().numpy(), gs.cpu().numpy(), tok.cpu().numpy(), 4)
     close(got.cpu().numpy(), ref, "fp4_gemm_tc 64-pair groups")
-    # grouped_fp4_gemm: 300 pairs, a popular expert (> 64 pairs: split into tiles), repeated output rows, ids out of range
+    sizes = [128, 100, 65, 17]                                              # the same on the 128-pair tile
+    gs = torch.tensor(np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32), device=DEV)
+    P = int(sum(sizes))
+    tok = torch.from_numpy(rng.integers(0, X, P).astype(np.int32)).to(DEV)
+    got = hipkern.fp4_gemm_tc(hipkern.permute_x(x), wtl, stl, ge, gs, tok, P, 128)
+    ref = O.grouped_gemm(bf16_vals(x), w.cpu().numpy(), s.cpu().numpy(), ge.cpu().numpy(), gs.cpu().numpy(), tok.cpu().numpy(), 4)
+    close(got.cpu().numpy(), ref, "fp4_gemm_tc 128-pair groups")
+    # grouped_fp4_gemm: 300 pairs, a popular expert (> 128 pairs: a 256-pair tile), repeated output rows, ids out of range
     P2 = 300
     eid = rng.choice(E, P2, p=[0.5, 0.1, 0.1, 0.1, 0.1, 0.1]).astype(np.int32)
     eid[[7, 100]] = [-1, E]                                                 # dropped by the dispatch
@@ -842,6 +849,36 @@ def test_prefill_layer_vs_oracle():
     close(y.cpu().numpy(), ref, "prefill layer I=1664")
 
 
+@pytest.mark.parametrize("tiled", [True, False])
+def test_prefill_long_k_loops_on_the_larger_tiles(tiled):
+    """Many pairs per expert at hidden 7168: groups of exactly 128 and 256 pairs, of 129 and of less than a token block on the 128- and
+    256-pair tiles with 56-step k-loops (w13), against the oracle as in test_prefill_stages_vs_oracle; w2 (I = 1664, 13 steps)
+    from the kernel's own h."""
+    from dsv41_amd import moe, quant
+    E, H, I, k = 4, 7168, 1664, 1
+    counts = [256, 128, 129, 256 + 9]
+    T = sum(counts)
+    ws = make_experts(E, H, I, 620 + int(tiled))
+    ex = to_ex(*ws, tiled)
+    rng = np.random.default_rng(15)
+    eid = rng.permutation(np.repeat(np.arange(E), counts)).astype(np.int32)[:, None]
+    wt = (0.5 + rng.random((T, k))).astype(np.float32)
+    xq = quant.fake_quant_fp8(rand_x(T, H, 16).to(DEV))
+    st = moe.prefill_up(xq, torch.from_numpy(eid).to(DEV), torch.from_numpy(wt).to(DEV), ex, 10.0)
+    ge, gs = st.grp_expert.cpu().numpy(), st.grp_start.cpu().numpy()
+    G = int(np.count_nonzero(ge >= 0))
+    assert not st.light and sorted(np.diff(gs[:G + 1])) == [9, 128, 129, 256, 256]
+    W13, S13, W2, S2 = [w.cpu().numpy() for w in ws]
+    gu = O.grouped_gemm(bf16_vals(xq), W13, S13, ge, gs, st.tok_sorted.cpu().numpy(), G)
+    h_ref = O.swiglu_quant(gu, st.wt_sorted.cpu().numpy(), I, 10.0)
+    h = _e4m3_values(st.hc, st.hs)
+    diff = h != h_ref
+    assert diff.mean() < 2e-3, f"{diff.mean():.2e} of h differs"
+    assert np.all(np.abs(h - h_ref)[diff] <= np.abs(h_ref)[diff] * 0.25 + 2.0 ** -9 * np.abs(h_ref).max())
+    moe.prefill_down(st, ex)
+    close(st.y2.cpu().numpy(), O.grouped_gemm(h, W2, S2, ge, gs, np.arange(T, dtype=np.int32), G), f"w2 after long k-loops tiled={tiled}")
+
+
 # ------------------------------------------------------------------------------------------ benchmark configs at full shape
 def test_configs0_single_gemv_full_shape():
     """one FP4 GEMV, W [2048 x 4096] E2M1 (uniform nibbles), E8M0 scale bytes 119..123, x [1 x 4096] N(0,1)
@@ -869,8 +906,8 @@ def test_configs0_single_gemv_full_shape():
 
 def test_configs3_prefill_full_shape(full_layer):
     """2048 tokens x top-8 over 384 experts with Zipf(1.1) popularity (the benchmark's own routing),
-    hidden 7168, intermediate 1664, tiled weights: every expert touched, the busiest spread over many 128-pair groups
-    (56-step k-loops). Sampled tokens (including tokens of the busiest expert) against the oracle, and against the
+    hidden 7168, intermediate 1664, tiled weights: every expert touched, the busiest spread over many 64-pair groups
+    (43 pairs per expert: the light tile; 56-step k-loops). Sampled tokens (including tokens of the busiest expert) against the oracle, and against the
     decode path on the same token."""
     from bench import zipf_routing
     from dsv41_amd import moe, quant
