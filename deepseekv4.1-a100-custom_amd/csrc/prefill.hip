@@ -322,39 +322,8 @@ __device__ __forceinline__ void prefill_item128(const PrefillArgs& a, const int 
             for (int u = 0; u < 4; ++u) {
                 if (!tb_on[u]) continue;   // wave-uniform: no pair of this token block is in the group
                 const int pr = 64 * ph + 16 * u + col;
-                float h[2][4];
-                float mx = 0.f;
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const float gv[4] = {acc[j][u].x, acc[j][u].y, acc[j][u].z, acc[j][u].w};
-                    const float uv[4] = {acc[2 + j][u].x, acc[2 + j][u].y, acc[2 + j][u].z, acc[2 + j][u].w};
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        float gg = gv[i], uu = uv[i];
-                        if (a.limit > 0.f) {
-                            uu = fminf(fmaxf(uu, -a.limit), a.limit);
-                            gg = fminf(gg, a.limit);
-                        }
-                        float hv = gg * (1.0f / (1.0f + expf(-gg))) * uu;
-                        hv = bf16_round(hv * wgt[u]);
-                        h[j][i] = hv;
-                        mx = fmaxf(mx, fabsf(hv));
-                    }
-                }
-                // the 32 columns of pair pr sit in the 4 lanes col + 16 kb: one FP8 group
-                mx = fmaxf(mx, __shfl_xor(mx, 16));
-                mx = fmaxf(mx, __shfl_xor(mx, 32));
-                const int ex = fq8_exponent(mx);
-                if (pr < m) {
-                    const long long p = p0 + pr;
-                    const int c0 = cb * 128 + 32 * cg;
-#pragma unroll
-                    for (int j = 0; j < 2; ++j) {
-                        const uint32_t codes = fq8_code4_hw(h[j][0], h[j][1], h[j][2], h[j][3], ex);
-                        *(gmem_u32*)(a.hc + p * a.ldhc + c0 + 16 * j + 4 * kb) = codes;
-                    }
-                    if (kb == 0) *(gmem_u8*)(a.hs + p * a.ldhs + (c0 >> 5)) = (uint8_t)(ex + 127);
-                }
+                const v4f gt[2] = {acc[0][u], acc[1][u]}, up[2] = {acc[2][u], acc[3][u]};
+                swiglu_store(a, gt, up, wgt[u], pr < m, (long long)p0 + pr, cb * 128 + 32 * cg, kb);
             }
         } else {
 #pragma unroll
@@ -718,38 +687,8 @@ __device__ __forceinline__ void prefill_item256(const PrefillArgs& a, const int 
             for (int u = 0; u < 8; ++u) {
                 if (!tb_on[u]) continue;
                 const int pr = 16 * (2 * u + ph) + col;
-                float h[2][4];
-                float mx = 0.f;
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const float gv[4] = {acc[j][u].x, acc[j][u].y, acc[j][u].z, acc[j][u].w};
-                    const float uv[4] = {acc[2 + j][u].x, acc[2 + j][u].y, acc[2 + j][u].z, acc[2 + j][u].w};
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        float gg = gv[i], uu = uv[i];
-                        if (a.limit > 0.f) {
-                            uu = fminf(fmaxf(uu, -a.limit), a.limit);
-                            gg = fminf(gg, a.limit);
-                        }
-                        float hv = gg * (1.0f / (1.0f + expf(-gg))) * uu;
-                        hv = bf16_round(hv * wgt[u]);
-                        h[j][i] = hv;
-                        mx = fmaxf(mx, fabsf(hv));
-                    }
-                }
-                mx = fmaxf(mx, __shfl_xor(mx, 16));
-                mx = fmaxf(mx, __shfl_xor(mx, 32));
-                const int ex = fq8_exponent(mx);
-                if (pr < m) {
-                    const long long p = p0 + pr;
-                    const int c0 = cb * 128 + 32 * cg;
-#pragma unroll
-                    for (int j = 0; j < 2; ++j) {
-                        const uint32_t codes = fq8_code4_hw(h[j][0], h[j][1], h[j][2], h[j][3], ex);
-                        *(gmem_u32*)(a.hc + p * a.ldhc + c0 + 16 * j + 4 * kb) = codes;
-                    }
-                    if (kb == 0) *(gmem_u8*)(a.hs + p * a.ldhs + (c0 >> 5)) = (uint8_t)(ex + 127);
-                }
+                const v4f gt[2] = {acc[0][u], acc[1][u]}, up[2] = {acc[2][u], acc[3][u]};
+                swiglu_store(a, gt, up, wgt[u], pr < m, (long long)p0 + pr, cb * 128 + 32 * cg, kb);
             }
         } else {
 #pragma unroll
