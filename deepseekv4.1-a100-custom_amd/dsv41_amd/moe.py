@@ -354,7 +354,10 @@ def dense_gemv(W: torch.Tensor, x: torch.Tensor, out: torch.Tensor | None = None
 
 
 class PrefillState:
-    """Intermediates of the prefill path (sorted pair order): dispatch tables, h codes + E8M0, per-pair y2."""
+    """Intermediates of the prefill path (sorted pair order): dispatch tables, h codes + E8M0, per-pair y2. light: the groups hold
+    at most 64 pairs and take the light tile (a state that does not say so takes the larger ones, which compute any group)."""
+
+    light = False
 
     def __init__(self, **kw):
         self.__dict__.update(kw)

@@ -836,6 +836,20 @@ def test_prefill_stages_vs_oracle(tiled, limit, H):
     assert np.array_equal(out.view(torch.int16).cpu().numpy().view(np.uint16), O.f32_to_bf16_bits((y32.cpu().numpy() + bf16_vals(ys)).astype(np.float32)))
 
 
+def test_prefill_down_of_a_state_without_a_tile():
+    """A PrefillState that names its tables and h alone (no `light`) goes through the larger tiles, with the same bits."""
+    from dsv41_amd import moe, quant
+    E, H, I, k, T = 8, 512, 384, 2, 40
+    ex = to_ex(*make_experts(E, H, I, 640), True)
+    eid, wt = _skewed_routing(T, E, k, 2, 17)
+    xq = quant.fake_quant_fp8(rand_x(T, H, 18).to(DEV))
+    st = moe.prefill_up(xq, torch.from_numpy(eid).to(DEV), torch.from_numpy(wt).to(DEV), ex, 10.0)
+    y = moe.prefill_down(st, ex)
+    assert st.light
+    own = moe.PrefillState(**{n: v for n, v in vars(st).items() if n not in ("light", "y2")})
+    assert torch.equal(moe.prefill_down(own, ex), y) and bool(y.any())
+
+
 def test_prefill_layer_vs_oracle():
     """End to end at the benchmark's intermediate size (I = 1664, hidden 512, 16 experts, 300 tokens, top-8)."""
     from dsv41_amd import moe, quant
