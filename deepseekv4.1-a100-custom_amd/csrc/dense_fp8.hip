@@ -427,8 +427,9 @@ __global__ void __launch_bounds__(FS_THREADS) fp8_stream_kernel(const Fp8Args a,
 // activation bytes per weight byte through a CU's load path).
 // KH (up to 64 tokens in all, two chunks per stage): wave w takes 32 rows (w & 3) x all tokens of chunk w >> 2 of a stage; the
 // two k halves are added through LDS at the end. Otherwise (CS chunks per stage) 32 rows x half w >> 2 of the tokens.
-// One chunk per stage leaves room for two workgroups per CU, whose chains of barrier, operand reads, decoding and MFMAs
-// overlap: each chain is several times its MFMAs' time.
+// Bound by the chain of a k-step (barrier, operand reads, decoding, MFMAs), several times its MFMAs' time: about 0.35 us a
+// chunk with one workgroup on a CU. One chunk per stage leaves room for two, whose chains overlap and then take 0.57 us each; so
+// a K range of its own CU is worth more than sharing one, and sharing pays where ranges are long (hipkern.fp8_rows_plan).
 // With S > 1 the fp32 tiles of the ranges go to `part` and a second launch adds them in range order (few weight rows would
 // otherwise leave most CUs without a workgroup).
 // LDS: weights per chunk and 16-row block 1 KB (tiled: as stored, lane l's operand at 16 l; row-major: 16 rows x 64 B, row
@@ -686,6 +687,7 @@ static void fp8_launch(const Fp8Args& a, int tiled, hipStream_t st) {
     // few row blocks: 16 waves per workgroup so the K split still fills the CUs (not for 4 token tiles, whose
     // registers do not fit 16 waves per CU)
     const bool wide = MT <= 2 && nb < 256 && a.nk >= 64;
+    // (Figures of this kernel: fp8_stream_blocks gives most sizes past 8 tokens to the loader waves, which are faster there.)
     // >= 256 row blocks: two row blocks per 8-wave workgroup (every activation load feeds two weight tiles); one token
     // tile: 4 tiles in flight per wave, 3 when a wave has fewer than 4 chunks; two: 3; four: 2. Measured (median of 50
     // graph replays, against one row block per workgroup): 16 / 8 rows 5120 x 8192 20.4 -> 14.4 / 14.9 -> 12.0 us,

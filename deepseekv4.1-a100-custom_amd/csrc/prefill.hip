@@ -1313,9 +1313,9 @@ __global__ void __launch_bounds__(256) scatter_rows_kernel(const float* __restri
 }
 
 // The reference's grouped GEMM with its weighted output-row epilogue (moe_kernels.py:29-80, 155-200): y2[p] = codes(x)
-// [row] . deq(W[e_g])^T on the mixed 128 / 256-pair tile kernel (groups of up to 256 pairs), then out[row_out[p]] +=
-// fl(wt[p] * y2[p]) in a second launch (an epilogue of that form inside the tile kernel's k-loop made its compiled loop
-// twice as slow).
+// [row] . deq(W[e_g])^T on the mixed 128 / 256-pair tile kernel (groups of up to 256 pairs) or the light one (up to 64), then
+// out[row_out[p]] += fl(wt[p] * y2[p]) in a second launch (an epilogue of that form inside the mixed kernel's k-loop made its
+// compiled loop twice as slow; the light tile's comes after its k-loop and stores the rows of a new output itself, below).
 static int grouped_gemm_scatter(PrefillTile tile, const uint8_t* xc, long long ldx, const uint8_t* xs, long long ldxs, int x_rows,
                                               const uint8_t* xlc, const uint8_t* xls, const int* lo_flag,
                                               const int* row_of_pair, const uint8_t* W, long long stride_we, const uint8_t* S,

@@ -183,9 +183,10 @@ def grouped_gemm_scatter(xc: torch.Tensor, xs: torch.Tensor, w: torch.Tensor, s:
                          n_groups: int | None = None, y2: torch.Tensor | None = None, lo=None,
                          gmax: int = TILE_GROUP) -> torch.Tensor:
     """out[row_out[p]] += wt[p] * codes(x)[row_of_pair[p]] . deq(W[e_g])^T over the pairs p of the first n_groups
-    groups (<= gmax <= 256 pairs each, LIGHT_GROUP taking the light tile; default every table entry); distinct: device int32 scalar, non-zero when no two pairs
-    share an output row (then stores when not accum, else read-add-write; otherwise fp32 atomics); y2: fp32
-    [n_pairs, N] workspace (allocated when None); dsv41_fp4_grouped_gemm_scatter."""
+    groups (<= gmax <= 256 pairs each, LIGHT_GROUP taking the light tile; default every table entry); distinct: device int32
+    scalar, non-zero when no two pairs share an output row (then stores when not accum, else read-add-write; otherwise fp32
+    atomics); y2: fp32 [n_pairs, N] workspace (allocated when None; not written where the light tile stores the output rows
+    itself); dsv41_fp4_grouped_gemm_scatter / _scatter_g64."""
     dev = _lib.require_cuda(xc, xs, w, s, grp_expert, grp_start, row_of_pair, row_out, wt, distinct, out, y2)
     E, N, Kh = w.shape
     K = Kh * 2

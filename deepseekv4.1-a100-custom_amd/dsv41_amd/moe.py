@@ -500,8 +500,8 @@ def shared_expert(xq: torch.Tensor, Ws13: torch.Tensor, Ws2: torch.Tensor, limit
 
 def shared_expert_rows(xq: torch.Tensor, sh_w13, sh_w2, inter: int, limit: float) -> torch.Tensor:
     """bf16 ys = linear_w(swiglu_quant(linear_w(xq, sh_w13)), sh_w2) (decode.py:368-371, model.py:409-412) for
-    bf16 tensors or w8.W8 weights: the FP8 GEMM streams W8 weights (up to 64 rows per launch), the library GEMM takes
-    bf16 weights or more rows."""
+    bf16 tensors or w8.W8 weights, through w8.linear_w: the FP8 kernels read W8 weights up to some hundred rows, the library
+    GEMM takes bf16 weights or more rows."""
     from .fused import swiglu_quant
     from .w8 import linear_w
     gu = linear_w(xq, sh_w13)
@@ -586,12 +586,13 @@ class MoE:
     scaled), x fake-quantised to FP8 (model.py:565), the routed FP4 experts, the shared expert (bf16, or FP8 w8.W8 as
     the checkpoint stores it), and
     y = bf16(sum_j w_j y2_j + shared) (model.py:589-591).
-      * <= 16 tokens (decode): the router GEMV on fp32 weights as split-K partial sums with the FP8 quantisation of x, then the two fused decode
-        launches (routing inside the up launch for one token; a bf16 shared expert rides in both launches when it fits
-        them, else runs as its own launches first; an FP8 one runs first as two FP8 GEMM launches and a SwiGLU);
-      * > 16 tokens (prefill): router logits and the shared expert's two products as plain library GEMMs (F.linear on
-        the GPU, as the reference runs them, model.py:392, 410-412; w8.py:102-103), gate_topk, then the prefill grouped
-        GEMMs with the slot-ordered combine.
+      * <= 16 tokens (decode): the router GEMV on fp32 weights as split-K partial sums with the FP8 quantisation of x, then
+        the two fused decode launches (routing inside the up launch for up to PAIRS_MAX_M tokens; a shared expert, bf16 or tiled
+        FP8, rides in both launches when it fits them, else runs as its own launches first: two GEMMs and a SwiGLU);
+      * > 16 tokens (prefill): router logits as a plain library GEMM (F.linear on the GPU, as the reference runs it,
+        model.py:392), the shared expert's two products by w8.linear_w (bf16 weights: library GEMMs, model.py:410-412; FP8
+        weights: the FP8 kernels up to some hundred rows, then library GEMMs on the dequantised weights), gate_topk, then
+        the prefill grouped GEMMs with the slot-ordered combine.
     Attribute names follow the reference (n_experts, topk, score_func, gate_temp, norm_topk_prob, route_scale,
     swiglu_limit, gate_w, gate_bias, inter, sh_w13, sh_w2). Routing of the last call: last_routing. The output and the routing
     are the call's own tensors at every size; up to 16 tokens the work between shares its buffers (the module's docstring)."""

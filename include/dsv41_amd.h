@@ -242,7 +242,8 @@ int dsv41_fp4_grouped_gemm_scatter(const uint8_t* xc, long long ldx, const uint8
                                    float* out, long long ldo, int out_rows, float* y2, long long ldy2, void* stream);
 
 /* dsv41_fp4_grouped_gemm_scatter for groups of <= 64 pairs, on the 64-pair tile (larger groups, of which the first 256
- * pairs are computed, in passes of 64). */
+ * pairs are computed, in passes of 64). With accum = 0, distinct rows and no second term (xlc NULL, or *lo_flag 0) the tile
+ * stores fl(wt * row) into out itself and leaves y2 unwritten; the same values. */
 int dsv41_fp4_grouped_gemm_scatter_g64(const uint8_t* xc, long long ldx, const uint8_t* xs, long long ldxs, int x_rows,
                                    const uint8_t* xlc, const uint8_t* xls, const int* lo_flag, const int* row_of_pair, const uint8_t* W, long long stride_we, const uint8_t* S,
                                    long long stride_se, int tiled, int E, int N, int K, const int* grp_expert, const int* grp_start,
