@@ -886,7 +886,14 @@ extern "C" int dsv41_dequant_fp8(const uint8_t* W, long long ldw, int tiled, con
                                  uint16_t* out, long long ldo, void* stream) {
     if (!W || !S || !out || N <= 0 || K <= 0 || (K & 15) || ldo < K || lds < (K + 31) / 32) return DSV41_EINVAL;
     if (tiled ? ((N & 15) || (K & 63) || ldw != K) : ldw < K) return DSV41_EINVAL;
-    const long long wgs = (((long long)N + 15) / 16) * (((long long)K + 255) / 256);
-    dequant_fp8_kernel<<<(unsigned)wgs, 256, 0, (hipStream_t)stream>>>(W, ldw, tiled, S, lds, N, K, out, ldo);
-    return (int)hipGetLastError();
+    // a launch takes fewer than 2^32 threads: rows beyond that go to launches of their own
+    const long long ncb = ((long long)K + 255) / 256, step = max((1ll << 23) / ncb * 16 & ~31ll, 32ll);
+    for (long long n0 = 0; n0 < N; n0 += step) {
+        const long long rows = min(step, N - n0);
+        dequant_fp8_kernel<<<(unsigned)((rows + 15) / 16 * ncb), 256, 0, (hipStream_t)stream>>>(W + n0 * (tiled ? K : ldw), ldw, tiled, S + n0 / 32 * lds, lds,
+                                                                                          (int)rows, K, out + n0 * ldo, ldo);
+        const hipError_t err = hipGetLastError();
+        if (err != hipSuccess) return (int)err;
+    }
+    return 0;
 }

@@ -82,6 +82,21 @@ def test_dequant_fp8_shapes(N, K, tiled, pad):
     assert np.array_equal(np.isnan(O.bf16_bits_to_f32(got)), nan) and np.array_equal(got[~nan], ref[~nan])
 
 
+def test_dequant_fp8_more_rows_than_one_launch_takes():
+    """2^28 rows of 16 (a workgroup per 16 rows: 2^32 threads) in launches of 2^27: the rows either side of each launch's end."""
+    from dsv41_amd import quant
+    N, K = (1 << 28) + 48, 16
+    g = torch.Generator(device=DEV).manual_seed(29)
+    w = torch.randint(0, 128, (N // 8, 16), generator=g, dtype=torch.int64, device=DEV).view(torch.uint8).view(N, K)
+    s = torch.randint(100, 140, ((N + 31) // 32, 1), generator=g, dtype=torch.uint8, device=DEV)
+    got = quant.dequant_fp8_block(w, s)
+    for n0 in (0, (1 << 27) - 64, 1 << 27, (1 << 28) - 64, N - 48):
+        rows = slice(n0, n0 + 48)
+        ref = quant.dequant_fp8_block(w[rows].clone(), s[n0 // 32:n0 // 32 + 2].clone())
+        assert torch.equal(got[rows].view(torch.int16), ref.view(torch.int16)), n0
+        assert bool(ref.any())
+
+
 @pytest.mark.parametrize("tiled", [False, True])
 @pytest.mark.parametrize("rows,N", [(4, 256), (16, 256), (64, 256), (16, 4112)])
 def test_fp8_gemm_decode_one_hot_exact(tiled, rows, N):
