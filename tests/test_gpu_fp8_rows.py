@@ -87,6 +87,26 @@ def test_fp8_gemm_rows(M, N, K, tiled):
         assert bad(floats=2 * M * N - 1) == -1
 
 
+@pytest.mark.parametrize("M", [40, 70, 400])
+def test_every_code_and_scale(M):
+    """Each E4M3 code (NaN among them) under each scale byte 0 .. 255 (products below the normal range, infinities), picked by one-hot
+    rows on the loader-wave kernel and both tile heights: the dequantised weight, as the library product of it gives it. A NaN
+    or infinite weight makes NaN of its whole row (0 times it) on either side."""
+    from dsv41_amd import hipkern, w8
+    K, N, c0 = 1024, 256 * 32, 8 * (M // 10)
+    code = 8 * (torch.arange(N) % 32)[:, None] + torch.arange(8)
+    w = torch.zeros(N, K, dtype=torch.uint8)
+    w[:, c0:c0 + 8] = code.to(torch.uint8)            # row n of a scale block: codes 8 (n % 32) ..
+    W = w8.W8(w.to(DEV), torch.arange(256, dtype=torch.uint8)[:, None].expand(256, K // 32).contiguous().to(DEV))
+    assert M <= 64 or hipkern.fp8_rows_plan(M, N, K) == ((64, 1) if M == 70 else (128, 1))
+    x = torch.zeros(M, K, dtype=torch.bfloat16, device=DEV)
+    for j in range(8):
+        x[M - 1 - j, c0 + j] = 1.0
+    y, lib = w8.linear_w(x, W), torch.nn.functional.linear(x, W.bf16())
+    assert torch.equal(y.isnan(), lib.isnan()) and torch.equal(y[~y.isnan()], lib[~lib.isnan()])
+    assert bool(y.isnan().any()) and bool((y == 0).any()) and bool((y.abs() > 1e38).any())
+
+
 def test_linear_w_rows_plan_and_watchers():
     """linear_w past 64 rows: the tiles give the library route's values; calls that something watches keep the library."""
     from dsv41_amd import hipkern, w8
